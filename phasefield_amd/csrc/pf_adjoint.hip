@@ -732,7 +732,8 @@ template <int K, int P, int NF, bool NOF> struct Adj {
         const unsigned *keep = vec && mby ? sd.count : nullptr;
         hipLaunchKernelGGL(adj_list_flag_kernel, dim3(gb), dim3(256), 0, st, sd.flag, N);
         hipLaunchKernelGGL(general_count_kernel, dim3(nl), dim3(256), 0, st, sd.flag, keep, N,
-                           ablock, ListOrder{}, static_cast<int *>(nullptr));
+                           ablock, ListOrder{}, static_cast<int *>(nullptr),
+                           static_cast<uint32_t *>(nullptr));
         hipLaunchKernelGGL(general_scan_kernel, dim3(1), dim3(1024), 0, st, ablock, int(nl),
                            static_cast<int *>(nullptr));
         hipLaunchKernelGGL(general_scatter_kernel, dim3(nl), dim3(256), 0, st, sd.flag, keep, N,
@@ -745,15 +746,15 @@ template <int K, int P, int NF, bool NOF> struct Adj {
           if (vec && mby == 8)
             hipLaunchKernelGGL((diffuse_bulk_march_kernel<FormF64, P, NF, NOF, 8, 2, 1>),
                                dim3(mnb), dim3(64, 8), 0, st, lam_c, lam_c2, sd.count, dc, v.nx,
-                               v.ny, v.nz, mzc, mtx, mty, int(mnb));
+                               v.ny, v.nz, mzc, mtx, mty, int(mnb), (s & 1) != 0);
           else if (vec && mby == 16)
             hipLaunchKernelGGL((diffuse_bulk_march_kernel<FormF64, P, NF, NOF, 16, 2, 1>),
                                dim3(mnb), dim3(64, 16), 0, st, lam_c, lam_c2, sd.count, dc, v.nx,
-                               v.ny, v.nz, mzc, mtx, mty, int(mnb));
+                               v.ny, v.nz, mzc, mtx, mty, int(mnb), (s & 1) != 0);
           else if (vec && mby == 32)
             hipLaunchKernelGGL((diffuse_bulk_march_kernel<FormF64, P, NF, NOF, 32, 2, 2>),
                                dim3(mnb), dim3(64, 16), 0, st, lam_c, lam_c2, sd.count, dc, v.nx,
-                               v.ny, v.nz, mzc, mtx, mty, int(mnb));
+                               v.ny, v.nz, mzc, mtx, mty, int(mnb), (s & 1) != 0);
           else if (vec)
             hipLaunchKernelGGL((diffuse_bulk_vec_kernel<FormF64, P, NF, NOF, 4, 2>),
                                dim3(gvec.nblocks), dim3(64, 4), 0, st, lam_c, lam_c2, sd.flag, dc,

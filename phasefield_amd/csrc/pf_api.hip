@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "../../include/phasefield_amd.h"
+#include "pf_diffuse_direct.h"
 #include "pf_handle_access.h"
 #include "pf_kernels.h"
 
@@ -68,6 +69,10 @@ struct pf_handle {
   uint8_t *unit = nullptr;   // scratch of the classification: per-cell unit-vector phase
   unsigned *bulk_count = nullptr;  // [4] bulk cells per phase of the last classification
   bool flag_valid = false;   // flags describe the current value_phase and stencil
+  bool list_stale = false;   // flags newer than the diffusion list built from them
+  bool len_stale = false;    // flags newer than the length pf_list_lengths reports
+  uint32_t *packed = nullptr;  // the bulk flags, two bits per cell (direct kernel)
+  bool diff_direct = true;   // single sub-steps in one launch (use_direct)
   bool unit_valid = false;   // unit bytes describe the current value_phase and bulk_mask
   int flag_nf = 0;           // stencil faces the flags were computed for
   int diff_by = -1;          // rows of the bulk diffusion tile (0: storage order, -1: by size)
@@ -77,6 +82,7 @@ struct pf_handle {
   bool diff_march = true;    // ... in its plane-marching form
   int march_by = 0;          // its tile rows and z-chunk, picked by timing at first use
   int march_zc = 0;
+  bool flip = false;         // direction of the next bulk pass (alternates)
   int *list_len = nullptr;   // [0]: cells the last sweep listed, [1]: cells the diffusion lists
   int *ccount = nullptr;     // pair lists: listed cells per list block ([nblocks + 1])
   bool ccount_pending = false;  // ccount not yet summed into list_len[1]
@@ -297,7 +303,7 @@ hipError_t launch_sweep(pf_handle *h, const PFConsts<typename F::A> &cs) {
     const ListOrder order = sweep_list_order(h);
     hipLaunchKernelGGL(general_count_kernel, dim3(nl), dim3(256), 0, h->stream, h->sflag,
                        static_cast<const unsigned *>(nullptr), h->N, h->gblock, order,
-                       static_cast<int *>(nullptr));
+                       static_cast<int *>(nullptr), static_cast<uint32_t *>(nullptr));
     hipLaunchKernelGGL(general_scan_kernel, dim3(1), dim3(1024), 0, h->stream, h->gblock, int(nl),
                        h->list_len);
     hipLaunchKernelGGL(general_scatter_kernel, dim3(nl), dim3(256), 0, h->stream, h->sflag,
@@ -421,18 +427,16 @@ hipError_t launch_march(pf_handle *h, const DiffConsts<typename F::A> &dc,
     const int tiles_x = (nx + 64 * V - 1) / (64 * V), tiles_y = (ny + by - 1) / by;
     const long nblocks = long(tiles_x) * tiles_y * ((nz + zc - 1) / zc);
     if (nblocks > 0x7fffffffL) return hipErrorInvalidConfiguration;
-    if (by == 8)
-      hipLaunchKernelGGL((diffuse_bulk_march_kernel<F, P, NF, NOF, 8, V, 1>), dim3(nblocks),
-                         dim3(64, 8), 0, h->stream, cin, cout, h->bulk_count, dc, nx, ny, nz, zc,
-                         tiles_x, tiles_y, int(nblocks));
-    else if (by == 16)
-      hipLaunchKernelGGL((diffuse_bulk_march_kernel<F, P, NF, NOF, 16, V, 1>), dim3(nblocks),
-                         dim3(64, 16), 0, h->stream, cin, cout, h->bulk_count, dc, nx, ny, nz, zc,
-                         tiles_x, tiles_y, int(nblocks));
-    else  // 32 rows: two per wavefront
-      hipLaunchKernelGGL((diffuse_bulk_march_kernel<F, P, NF, NOF, 32, V, 2>), dim3(nblocks),
-                         dim3(64, 16), 0, h->stream, cin, cout, h->bulk_count, dc, nx, ny, nz, zc,
-                         tiles_x, tiles_y, int(nblocks));
+    auto go = [&](auto rows, auto per_wave) {
+      constexpr int BY = decltype(rows)::value, R = decltype(per_wave)::value;
+      hipLaunchKernelGGL((diffuse_bulk_march_kernel<F, P, NF, NOF, BY, V, R>), dim3(nblocks),
+                         dim3(64, BY / R), 0, h->stream, cin, cout, h->bulk_count, dc, nx, ny, nz,
+                         zc, tiles_x, tiles_y, int(nblocks), h->flip);
+    };
+    using std::integral_constant;
+    if (by == 8) go(integral_constant<int, 8>(), integral_constant<int, 1>());
+    else if (by == 16) go(integral_constant<int, 16>(), integral_constant<int, 1>());
+    else go(integral_constant<int, 32>(), integral_constant<int, 2>());  // two rows per wavefront
     return hipGetLastError();
   };
   if (h->march_by == 0) {
@@ -504,7 +508,77 @@ hipError_t launch_march(pf_handle *h, const DiffConsts<typename F::A> &dc,
       }
     }
   }
-  return launch(h->march_by, h->march_zc);
+  const hipError_t e = launch(h->march_by, h->march_zc);
+  h->flip = !h->flip;  // the next sub-step starts where this one ended
+  return e;
+}
+
+// whether the single sub-steps run the plane-marching kernel (which addresses a plane with 32-bit
+// byte offsets)
+template <class F> bool use_march(const pf_handle *h) {
+  constexpr int V = F::kMixed ? 4 : 2;  // 16-byte runs per lane
+  return h->diff_split && h->diff_vec && h->diff_march && h->d.nx % V == 0 &&
+         long(h->d.nx) * h->d.ny * long(sizeof(typename F::C)) < (1L << 32) &&
+         (h->diff_by < 0 || h->diff_by == 8 || h->diff_by == 16 || h->diff_by == 32);
+}
+
+// whether none of the pins that select another diffusion kernel is set
+bool default_diffusion(const pf_handle *h) {
+  return h->diff_variant == 0 && h->diff_split && h->diff_vec && h->diff_march && h->diff_by < 0 &&
+         h->diff_zchunk_override == 0;
+}
+// Whether they run as one launch of the direct kernel: rows the marching kernel does not take, and
+// domains whose two concentration buffers are at most half of the memory-side cache.  Per step, one
+// domain on the GPU / each of three in turn, marching + listed pass against the direct kernel:
+//   128^3 FP64 (34 MB)    3.37 / 2.30 ms against 1.88 / 1.55
+//   192^3 mixed (64 MB)   6.36 / 3.95    against 3.67 / 3.05
+//   192^3 FP64 (113 MB)   8.61 / 5.75    against 4.80 / 6.18
+//   224^3 FP64 (180 MB)  11.29 / 8.56    against 7.31 / 10.01
+//   256^3 FP64 (268 MB)  14.29 / 12.39   against 12.92 / 14.58
+// Beyond half of the cache a second domain's passes push the first one's out between two sub-steps.
+bool use_direct(const pf_handle *h, int nf) {
+  if (!h->diff_direct || nf != 6 || h->d.nz == 1 || !default_diffusion(h)) return false;
+  const bool march = is_mixed(h) ? use_march<FormMixed>(h) : use_march<FormF64>(h);
+  return !march || 2 * h->cbuf <= size_t(128) << 20;
+}
+
+// the bulk flags of the current value_phase
+template <class T, int P, int NF, bool NOF> hipError_t ensure_flags(pf_handle *h) {
+  if (h->flag_valid && h->flag_nf == NF) return hipSuccess;
+  const hipError_t e = launch_classify<T, P, NF, NOF>(
+      h->stream, static_cast<const T *>(h->pfrac), h->unit, h->flag, h->d.nx, h->d.ny, h->d.nz, h->N,
+      h->bulk_mask, h->bulk_count, h->unit_valid);
+  if (e != hipSuccess) return e;
+  h->unit_valid = true;
+  h->flag_valid = true;
+  h->flag_nf = NF;
+  h->list_stale = true;
+  h->len_stale = true;
+  return hipSuccess;
+}
+
+// the list of the cells a single sub-step's bulk kernel leaves, from the flags
+template <class F> void build_list(pf_handle *h, int nf) {
+  // the plane-marching kernel leaves every cell whose flag is not its bulk phase; the other bulk
+  // kernels leave the flag-0 cells
+  const bool direct = use_direct(h, nf);
+  const unsigned *keep = use_march<F>(h) && !direct ? h->bulk_count : nullptr;
+  const unsigned nl = list_blocks(h->N);
+  // mixed: entries are byte pairs of cells (their codes share a byte); the count kernel keeps
+  // per-block counts of the listed cells, summed into list_len[1] when they are asked for
+  // (pf_list_lengths); FP64: list_len[1] is the list's length
+  ListOrder order;
+  order.pairs = F::kMixed;
+  int *cells = F::kMixed && !direct ? h->ccount : nullptr;
+  hipLaunchKernelGGL(general_count_kernel, dim3(nl), dim3(256), 0, h->stream, h->flag, keep, h->N,
+                     h->gblock, order, cells, direct ? h->packed : static_cast<uint32_t *>(nullptr));
+  hipLaunchKernelGGL(general_scan_kernel, dim3(1), dim3(1024), 0, h->stream, h->gblock, int(nl),
+                     F::kMixed || direct ? static_cast<int *>(nullptr) : h->list_len + 1);
+  hipLaunchKernelGGL(general_scatter_kernel, dim3(nl), dim3(256), 0, h->stream, h->flag, keep, h->N,
+                     h->gblock, h->glist, order);
+  h->ccount_pending = F::kMixed && !direct;
+  h->len_stale = direct;
+  h->list_stale = false;
 }
 
 // one sub-step from `cin` into `cout` with the handle's kernel choice and bulk flags
@@ -521,38 +595,17 @@ hipError_t launch_diffuse_io(pf_handle *h, const DiffConsts<typename F::A> &dc,
   } else {
     const unsigned nb = blocks_for(h->N);
     constexpr int V = F::kMixed ? 4 : 2;  // 16-byte runs per lane
-    // (the marching kernel addresses a plane with 32-bit byte offsets)
-    const bool march = h->diff_split && h->diff_vec && h->diff_march && h->d.nx % V == 0 &&
-                       long(h->d.nx) * h->d.ny * long(sizeof(typename F::C)) < (1L << 32) &&
-                       (h->diff_by < 0 || h->diff_by == 8 || h->diff_by == 16 || h->diff_by == 32);
-    if (!h->flag_valid || h->flag_nf != NF) {
-      const hipError_t ec =
-          launch_classify<T, P, NF, NOF>(h->stream, pf, h->unit, h->flag, h->d.nx, h->d.ny,
-                                         h->d.nz, h->N, h->bulk_mask, h->bulk_count,
-                                         h->unit_valid);
-      if (ec != hipSuccess) return ec;
-      h->unit_valid = true;
-      if (h->diff_split) {
-        // the plane-marching kernel leaves every cell whose flag is not its bulk phase; the other
-        // bulk kernels leave the flag-0 cells
-        const unsigned *keep = march ? h->bulk_count : nullptr;
-        const unsigned nl = list_blocks(h->N);
-        // mixed: entries are byte pairs of cells (their codes share a byte); the count kernel
-        // keeps per-block counts of the listed cells, summed into list_len[1] when they are asked
-        // for (pf_list_lengths); FP64: list_len[1] is the list's length
-        ListOrder order;
-        order.pairs = F::kMixed;
-        int *cells = F::kMixed ? h->ccount : nullptr;
-        hipLaunchKernelGGL(general_count_kernel, dim3(nl), dim3(256), 0, h->stream, h->flag, keep,
-                           h->N, h->gblock, order, cells);
-        hipLaunchKernelGGL(general_scan_kernel, dim3(1), dim3(1024), 0, h->stream, h->gblock,
-                           int(nl), F::kMixed ? static_cast<int *>(nullptr) : h->list_len + 1);
-        hipLaunchKernelGGL(general_scatter_kernel, dim3(nl), dim3(256), 0, h->stream, h->flag,
-                           keep, h->N, h->gblock, h->glist, order);
-        h->ccount_pending = F::kMixed;
+    const bool march = use_march<F>(h);
+    const hipError_t ec = ensure_flags<T, P, NF, NOF>(h);
+    if (ec != hipSuccess) return ec;
+    if (h->diff_split && h->list_stale) build_list<F>(h, NF);
+    if constexpr (NF == 6) {
+      if (use_direct(h, NF)) {
+        h->flip = !h->flip;  // the next sub-step starts where this one ends
+        return launch_direct<F, P, NOF>(h->stream, cin, cout, pf, h->packed, h->glist,
+                                        h->gblock + list_blocks(h->N), dc, h->d.nx, h->d.ny, h->d.nz,
+                                        h->flip);
       }
-      h->flag_valid = true;
-      h->flag_nf = NF;
     }
     auto go = [&](auto by, auto split) {
       constexpr int BY = decltype(by)::value;
@@ -708,6 +761,7 @@ void free_all(pf_handle *h) {
   if (h->squeue) hipFree(h->squeue);
   if (h->olist) hipFree(h->olist);
   if (h->gblock) hipFree(h->gblock);
+  if (h->packed) hipFree(h->packed);
   if (h->red) hipFree(h->red);
   for (int k = 0; k < 3; ++k)
     for (auto &pr : h->ev[k]) {
@@ -783,6 +837,7 @@ int pf_create(const pf_desc *desc, pf_handle **out) {
   if (const char *e = std::getenv("PFAMD_DIFF_SPLIT")) h->diff_split = std::atoi(e) != 0;
   if (const char *e = std::getenv("PFAMD_DIFF_VEC")) h->diff_vec = std::atoi(e) != 0;
   if (const char *e = std::getenv("PFAMD_DIFF_MARCH")) h->diff_march = std::atoi(e) != 0;
+  if (const char *e = std::getenv("PFAMD_DIFF_DIRECT")) h->diff_direct = std::atoi(e) != 0;
   if (const char *e = std::getenv("PFAMD_SWEEP_SPLIT")) h->sweep_split = std::atoi(e) != 0;
   if (const char *e = std::getenv("PFAMD_SWEEP_ROWS")) h->sweep_rows = std::atoi(e);
   if (const char *e = std::getenv("PFAMD_SWEEP_QUEUE")) h->sweep_queue = std::atoi(e) != 0;
@@ -807,6 +862,9 @@ int pf_create(const pf_desc *desc, pf_handle **out) {
     return rc;
   if ((rc = chk(hipMalloc(&h->flag, N), "alloc bulk flags")) != PF_OK) return rc;
   if ((rc = chk(hipMalloc(&h->unit, N), "alloc bulk flags")) != PF_OK) return rc;
+  if (use_direct(h.get(), h->NF) &&
+      (rc = chk(hipMalloc(&h->packed, (N + 15) / 16 * 4), "alloc packed flags")) != PF_OK)
+    return rc;
   if ((rc = chk(hipMalloc(&h->bulk_count, 4 * sizeof(unsigned)), "alloc bulk counts")) != PF_OK)
     return rc;
   if ((rc = chk(hipMalloc(&h->glist, N * 4), "alloc full-formula list")) != PF_OK) return rc;
@@ -1245,6 +1303,18 @@ int pf_list_lengths(pf_handle *h, int64_t *sweep_listed, int64_t *diffusion_list
   if (!h) return PF_ERR_INVALID;
   hipSetDevice(h->d.device);
   int v[2] = {0, 0};
+  if (h->len_stale) {  // the sub-steps since the flags were taken ran without that list
+    const bool march = is_mixed(h) ? use_march<FormMixed>(h) : use_march<FormF64>(h);
+    const unsigned nl = list_blocks(h->N);
+    hipLaunchKernelGGL(general_count_kernel, dim3(nl), dim3(256), 0, h->stream, h->flag,
+                       march ? h->bulk_count : static_cast<const unsigned *>(nullptr), h->N,
+                       h->ccount, ListOrder{}, static_cast<int *>(nullptr),
+                       static_cast<uint32_t *>(nullptr));
+    hipLaunchKernelGGL(general_scan_kernel, dim3(1), dim3(1024), 0, h->stream, h->ccount, int(nl),
+                       h->list_len + 1);
+    HIPCHK(h, hipGetLastError());
+    h->len_stale = false;
+  }
   if (h->ccount_pending) {  // the pair list's per-block cell counts, summed once
     hipLaunchKernelGGL(general_scan_kernel, dim3(1), dim3(1024), 0, h->stream, h->ccount,
                        int(list_blocks(h->N)), h->list_len + 1);

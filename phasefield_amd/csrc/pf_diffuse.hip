@@ -542,21 +542,6 @@ __device__ inline void store_codes4_nt(float *__restrict__ buf, long n, long i,
   __builtin_nontemporal_store(uint16_t(w), reinterpret_cast<uint16_t *>(comp_bytes(buf, n) + (i >> 1)));
 }
 
-template <class F, int V>
-__device__ inline void vec_update(const typename F::C *__restrict__ in, typename F::C *__restrict__ out,
-                                  long i, long n, const VecA<typename F::A, V> &c,
-                                  const typename F::A (&del)[V], const VecCode<V> &codes,
-                                  uint32_t key);
-template <>
-__device__ inline void vec_update<FormF64, 2>(const double *__restrict__, double *__restrict__ out,
-                                              long i, long, const VecA<double, 2> &c,
-                                              const double (&del)[2], const VecCode<2> &,
-                                              uint32_t) {
-  VecA<double, 2> o;
-  o.v[0] = c.v[0] + del[0];
-  o.v[1] = c.v[1] + del[1];
-  store_nt(reinterpret_cast<VecA<double, 2> *>(out + i), o);
-}
 // The mixed form's update of a run of four cells i..i+3: values stored at vdst, their four 4-bit
 // codes (one 16-bit word) at tdst; hbase = i * kCompCellMul gives the rounding hashes of comp_hash
 // by additions.
@@ -577,15 +562,21 @@ __device__ inline void run_update_mixed(float *__restrict__ vdst, uint16_t *__re
   store_nt(reinterpret_cast<VecA<float, 4> *>(vdst), o);
   __builtin_nontemporal_store(uint16_t(w), tdst);
 }
-template <>
-__device__ inline void vec_update<FormMixed, 4>(const float *__restrict__ in, float *__restrict__ out,
-                                                long i, long n, const VecA<float, 4> &c,
-                                                const float (&del)[4], const VecCode<4> &qi,
-                                                uint32_t key) {
-  run_update_mixed(out + i, reinterpret_cast<uint16_t *>(comp_bytes(out, n) + (i >> 1)), c, del,
-                   qi, key, uint32_t(i) * kCompCellMul);
+// The run's update, values at cell i of `out`.
+template <class F, int V>
+__device__ inline void vec_update(typename F::C *__restrict__ out, long i, long n,
+                                  const VecA<typename F::A, V> &c, const typename F::A (&del)[V],
+                                  const VecCode<V> &qi, uint32_t key) {
+  if constexpr (F::kMixed) {
+    run_update_mixed(out + i, reinterpret_cast<uint16_t *>(comp_bytes(out, n) + (i >> 1)), c,
+                         del, qi, key, uint32_t(i) * kCompCellMul);
+  } else {
+    VecA<double, 2> o;
+    o.v[0] = c.v[0] + del[0];
+    o.v[1] = c.v[1] + del[1];
+    store_nt(reinterpret_cast<VecA<double, 2> *>(out + i), o);
+  }
 }
-
 template <class F, int P, int NF, bool NOFLUX, int BY, int V>
 __global__ __launch_bounds__(64 * BY) void diffuse_bulk_vec_kernel(
     const typename F::C *__restrict__ cin, typename F::C *__restrict__ cout,
@@ -671,7 +662,7 @@ __global__ __launch_bounds__(64 * BY) void diffuse_bulk_vec_kernel(
           }
           del[v] = d.result(dc.r, Dp * dc.r);
         }
-        vec_update<F, V>(cin, cout, plane * (z + u) + oc, ncell, cc[u], del, qc[u], dc.key);
+        vec_update<F, V>(cout, plane * (z + u) + oc, ncell, cc[u], del, qc[u], dc.key);
       }
     }
   }
@@ -707,7 +698,7 @@ __global__ __launch_bounds__(64 * BY / R) void diffuse_bulk_march_kernel(
     const typename F::C *__restrict__ cin, typename F::C *__restrict__ cout,
     const unsigned *__restrict__ count, const DiffConsts<typename F::A> dc, const int nx,
     const int ny, const int nz, const int zchunk, const int tiles_x, const int tiles_y,
-    const int nblocks) {
+    const int nblocks, const bool flip) {
   using A = typename F::A;
   using VA = VecA<A, V>;
   static_assert(BY % R == 0, "rows per wavefront must divide the tile height");
@@ -727,7 +718,8 @@ __global__ __launch_bounds__(64 * BY / R) void diffuse_bulk_march_kernel(
   __shared__ VA s[2][BY][64];
   const int b = blockIdx.x;
   const int per = nblocks >> 3, rem = nblocks & 7, xcd = b & 7;
-  const int logical = xcd * per + (xcd < rem ? xcd : rem) + (b >> 3);
+  const int mine = per + (xcd < rem ? 1 : 0);
+  const int logical = xcd * per + (xcd < rem ? xcd : rem) + (flip ? mine - 1 - (b >> 3) : b >> 3);
   const int tx_t = logical % tiles_x;
   const int t2 = logical / tiles_x;
   const int ty_t = t2 % tiles_y;
@@ -896,8 +888,7 @@ __global__ __launch_bounds__(64 * BY / R) void diffuse_bulk_march_kernel(
           run_update_mixed(reinterpret_cast<float *>(vb), reinterpret_cast<uint16_t *>(tb),
                            pc.c[r], del, qc, dc.key, uint32_t(plane * z) * kCompCellMul + oh[r]);
         } else {
-          vec_update<F, V>(cin, reinterpret_cast<typename F::C *>(vb), 0, ncell, pc.c[r], del, qc,
-                           dc.key);
+          vec_update<F, V>(reinterpret_cast<typename F::C *>(vb), 0, ncell, pc.c[r], del, qc, dc.key);
         }
       }
       if (NF == 6) {
@@ -1217,13 +1208,26 @@ __global__ __launch_bounds__(256) void general_count_kernel(const uint8_t *__res
                                                             const unsigned *__restrict__ count,
                                                             long ncell, int *__restrict__ bcount,
                                                             const ListOrder order,
-                                                            int *__restrict__ cells) {
+                                                            int *__restrict__ cells,
+                                                            uint32_t *__restrict__ packed) {
   __shared__ int wsum[4];
   const long first = long(blockIdx.x) * (256L * kListChunk) + long(threadIdx.x) * kListChunk;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   __shared__ int csum[4];
   const int keep = count ? bulk_phase(count) : 0;
   const unsigned bits = listed_bits(flag, first, ncell, count, keep, order);
+  if (packed && first < ncell) {  // the flags of the 16 cells, two bits each (storage order)
+    uint32_t w = 0;
+    if (first + kListChunk <= ncell) {
+      const uint4 q = *reinterpret_cast<const uint4 *>(flag + first);
+      const uint32_t word[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+      for (int j = 0; j < kListChunk; ++j) w |= ((word[j >> 2] >> (8 * (j & 3))) & 3u) << (2 * j);
+    } else {
+      for (int j = 0; first + j < ncell; ++j) w |= (uint32_t(flag[first + j]) & 3u) << (2 * j);
+    }
+    packed[first / kListChunk] = w;
+  }
   int n = __popc(order.pairs ? pair_bits(bits) : bits);
   int nc = __popc(bits);
 #pragma unroll
@@ -1417,7 +1421,7 @@ PF_INST_CLASSIFY(float, 3)
 #define PF_INST_MARCH_ONE(F, P, NF, NOF, BY, V, R)                                                 \
   template __global__ void diffuse_bulk_march_kernel<F, P, NF, NOF, BY, V, R>(                     \
       const F::C *, F::C *, const unsigned *, const DiffConsts<F::A>, int, int, int, int, int,    \
-      int, int);
+      int, int, bool);
 #define PF_INST_MARCH_NF(F, P, BY, V, R)          \
   PF_INST_MARCH_ONE(F, P, 4, false, BY, V, R)     \
   PF_INST_MARCH_ONE(F, P, 6, false, BY, V, R)     \

@@ -89,7 +89,8 @@ __global__ void diffuse_bulk_march_kernel(const typename F::C *__restrict__ cin,
                                           const unsigned *__restrict__ count,
                                           const DiffConsts<typename F::A> dc, const int nx,
                                           const int ny, const int nz, const int zchunk,
-                                          const int tiles_x, const int tiles_y, const int nblocks);
+                                          const int tiles_x, const int tiles_y, const int nblocks,
+                                          const bool flip);
 
 template <class F, int P, int NF, bool NOFLUX>
 __global__ void diffuse_general_kernel(const typename F::C *__restrict__ cin,
@@ -174,11 +175,12 @@ __host__ __device__ inline bool id_row_breaks(uint64_t w, uint32_t G) {
   return b0 | (e0 & b1) | (e0 & e1 & b2) | (e0 & e1 & e2 & b3);
 }
 // `cells` (optional): the count kernel's per-block counts of listed cells, for lists whose
-// entries are not cells (pairs); general_scan_kernel over them gives the total
+// entries are not cells (pairs); general_scan_kernel over them gives the total.  `packed` (optional,
+// storage order): the flags two bits per cell, 16 cells per word.
 __global__ void general_count_kernel(const uint8_t *__restrict__ flag,
                                      const unsigned *__restrict__ count, long ncell,
                                      int *__restrict__ bcount, const ListOrder order,
-                                     int *__restrict__ cells);
+                                     int *__restrict__ cells, uint32_t *__restrict__ packed = nullptr);
 __global__ void general_scan_kernel(int *__restrict__ bcount, int nb,
                                     int *__restrict__ total_out);
 __global__ void general_scatter_kernel(const uint8_t *__restrict__ flag,

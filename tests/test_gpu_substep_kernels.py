@@ -1,0 +1,81 @@
+"""GPU: the diffusion sub-step kernels at the sizes where they can go wrong, bitwise against the
+oracle: rows of every remainder, odd plane counts, extents that wrap onto themselves, insulated z,
+every phase count and both forms, each on random states (nearly every cell listed) and on states
+that are bulk but for a few cells.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+from phasefield_amd import Domain
+from phasefield_amd._capi import PfParams
+from tests import helpers
+
+pytestmark = pytest.mark.gpu
+
+FORMS = [oracle.ORC_FP64, oracle.ORC_MIXED]
+
+
+@pytest.fixture(scope="module")
+def params(tmp_path_factory):
+    m = helpers.small_model(str(tmp_path_factory.mktemp("sk")), "fec_3d_256", nx=16, ny=16, nz=16,
+                            grains=4, nuclei=2)
+    q = oracle.as_orc_params(helpers.model_params(m))
+    q.diffusivity[0][2] = 5.0
+    return q
+
+
+def sparse_state(rng, nx, ny, nz, P):
+    """Ferrite with a slab of austenite and some mixed cells: bulk cells of both phases and a list."""
+    n = nx * ny * nz
+    ids, val = np.zeros((n, 4), np.int32), np.zeros((n, 4))
+    phase = np.zeros((n, 3))
+    gamma = np.arange(n) % nx < nx // 3
+    ids[:, 0] = np.where(gamma, 100001, 200001)
+    val[:, 0] = 1.0
+    phase[:, 0], phase[:, 1] = gamma, ~gamma
+    some = rng.choice(n, size=max(1, n // 40), replace=False)
+    w = 0.1 + 0.8 * rng.random(some.size)
+    ids[some, 0], ids[some, 1] = 100001, 200001
+    val[some, 0], val[some, 1] = w, 1.0 - w
+    phase[some] = 0.0
+    phase[some, 0], phase[some, 1] = w, 1.0 - w
+    if P == 3:
+        one = some[0]
+        ids[one, 0], val[one, 0], phase[one, 0], phase[one, 2] = 300001, w[0], 0.0, w[0]
+    return ids.reshape(-1), val.reshape(-1), phase.reshape(-1), 0.02 + 0.8 * rng.random(n)
+
+
+def check(shape, bc, P, form, state, params, counts):
+    nx, ny, nz = shape
+    q = PfParams.from_buffer_copy(params)
+    q.dims = 3 - (nz == 1) - (ny == 1)
+    g = Domain(nx, ny, nz, depth=4, nphase=P, precision="mixed" if form == oracle.ORC_MIXED else "fp64",
+               bc_z=bc)
+    g.set_params(q)
+    g.upload(*state)
+    o = oracle.OracleDomain(nx, ny, nz, 4, 1, form, bc)
+    o.set_params(oracle.as_orc_params(q))
+    o.set_state(*state)
+    for n in counts:
+        g.diffuse(0, n, q.dt_d[0])
+        o.diffuse(0, n, q.dt_d[0])
+    a, b = g.download(), o.get_state()
+    g.close()
+    assert np.array_equal(a["conc"], b["conc"])
+    if form == oracle.ORC_MIXED:
+        assert np.array_equal(a["conc_comp"], b["conc_comp"])
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("shape,bc,P", [((64, 20, 9), 0, 2), ((66, 7, 8), 1, 2), ((67, 9, 11), 0, 3),
+                                        ((33, 5, 3), 1, 2), ((128, 4, 2), 0, 3), ((3, 2, 5), 0, 2),
+                                        ((2, 3, 2), 1, 2), ((131, 6, 7), 1, 3)])
+def test_one_launch_substep_bitwise(shape, bc, P, form, params):
+    print(f"[gpu] one-launch sub-step {shape} bc={bc} P={P} form={form}", flush=True)
+    rng = np.random.default_rng(11)
+    check(shape, bc, P, form, sparse_state(rng, *shape, P), params, (1, 4))
+    ids, val, phase, conc = helpers.random_state(rng, *shape, 4, nphase=P)
+    check(shape, bc, P, form, (ids, val, phase, conc), params, (3,))
