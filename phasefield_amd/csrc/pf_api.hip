@@ -19,6 +19,7 @@
 
 #include "../../include/phasefield_amd.h"
 #include "pf_diffuse_direct.h"
+#include "pf_diffuse_tile.h"
 #include "pf_handle_access.h"
 #include "pf_kernels.h"
 
@@ -73,6 +74,8 @@ struct pf_handle {
   bool len_stale = false;    // flags newer than the length pf_list_lengths reports
   uint32_t *packed = nullptr;  // the bulk flags, two bits per cell (direct kernel)
   bool diff_direct = true;   // single sub-steps in one launch (use_direct)
+  bool diff_tile = true;     // several sub-steps per launch (tile_geom)
+  int tile_pin[3] = {0, 0, 0};  // PFAMD_DIFF_TILE=bx,by,steps
   bool unit_valid = false;   // unit bytes describe the current value_phase and bulk_mask
   int flag_nf = 0;           // stencil faces the flags were computed for
   int diff_by = -1;          // rows of the bulk diffusion tile (0: storage order, -1: by size)
@@ -686,6 +689,36 @@ hipError_t launch_diffuse(pf_handle *h, int s, const DiffConsts<typename F::A> &
   return e;
 }
 
+// Geometry of a launch of up to `left` sub-steps on independent planes, or false when the
+// single-sub-step kernels run.
+bool tile_geom(const pf_handle *h, int left, TileGeom &g) {
+  if (!h->diff_tile || !(h->NF == 4 || h->d.nz == 1) || !default_diffusion(h)) return false;
+  return tile_geometry(h->d.nx, h->d.ny, h->d.nz, left, h->tile_pin, g);
+}
+
+template <class F, int P, int NF, bool NOF>
+hipError_t launch_tile(pf_handle *h, int s, const DiffConsts<typename F::A> &dc,
+                       const TileGeom &g) {
+  using T = typename F::T;
+  using C = typename F::C;
+  const hipError_t e = ensure_flags<T, P, NF, NOF>(h);
+  if (e != hipSuccess) return e;
+  const int a = h->ccur[s], b = 1 - a;
+  hipLaunchKernelGGL((diffuse_tile_kernel<F, P>), dim3(unsigned(g.nblocks)), dim3(kTileNT), 0,
+                     h->stream, static_cast<const C *>(h->conc[s][a]),
+                     static_cast<C *>(h->conc[s][b]), static_cast<const T *>(h->pfrac), h->flag, dc,
+                     g, h->N, h->csub[s], s);
+  h->ccur[s] = b;
+  h->csub[s] += uint32_t(g.steps);
+  return hipGetLastError();
+}
+template <class F, int P>
+hipError_t dispatch_tile_p(pf_handle *h, int s, const DiffConsts<typename F::A> &dc,
+                           const TileGeom &g) {
+  if (h->NF == 4) return launch_tile<F, P, 4, false>(h, s, dc, g);
+  return launch_tile<F, P, 6, false>(h, s, dc, g);  // one plane: its z faces carry no flux
+}
+
 template <class F, int P>
 hipError_t dispatch_diffuse_p(pf_handle *h, int s, const DiffConsts<typename F::A> &dc) {
   if (h->NF == 4) return launch_diffuse<F, P, 4, false>(h, s, dc);
@@ -701,18 +734,28 @@ int run_diffuse(pf_handle *h, int s, int n, double factor) {
   // a change of tables with no sweep since: the first sub-step reads every cell's partition of
   // the previous tables; every cell is partitioned with the current tables after this batch
   if (!h->retable[s] && tables_differ(h, s)) h->retable[s] = 2;
-  // the first launch classifies bulk cells when the flags are stale; keep it out of the timing
-  dc.key = comp_step_key(h->csub[s]++, s);
-  hipError_t e = h->d.nphase == 2 ? dispatch_diffuse_p<F, 2>(h, s, dc)
-                                  : dispatch_diffuse_p<F, 3>(h, s, dc);
-  if (e != hipSuccess) return fail(h, PF_ERR_HIP, std::string("diffuse: ") + hipGetErrorString(e));
-  Timer t(h, 0, n - 1);
-  for (int it = 1; it < n; ++it) {
+  // one launch from sub-step `it` on; returns the sub-steps it did (0: an error)
+  hipError_t e = hipSuccess;
+  auto launch = [&](int it) -> int {
+    TileGeom g;
+    if (!h->retable[s] && tile_geom(h, n - it, g)) {
+      e = h->d.nphase == 2 ? dispatch_tile_p<F, 2>(h, s, dc, g) : dispatch_tile_p<F, 3>(h, s, dc, g);
+      return e == hipSuccess ? g.steps : 0;
+    }
     dc.key = comp_step_key(h->csub[s]++, s);
-    h->time_march = h->timing && it % kMarchTimingEvery == 0;
     e = h->d.nphase == 2 ? dispatch_diffuse_p<F, 2>(h, s, dc) : dispatch_diffuse_p<F, 3>(h, s, dc);
+    return e == hipSuccess ? 1 : 0;
+  };
+  // the first launch classifies bulk cells when the flags are stale; keep it out of the timing
+  const int first = launch(0);
+  if (!first) return fail(h, PF_ERR_HIP, std::string("diffuse: ") + hipGetErrorString(e));
+  Timer t(h, 0, n - first);
+  for (int it = first; it < n;) {
+    h->time_march = h->timing && it % kMarchTimingEvery == 0;
+    const int did = launch(it);
     h->time_march = false;
-    if (e != hipSuccess) return fail(h, PF_ERR_HIP, std::string("diffuse: ") + hipGetErrorString(e));
+    if (!did) return fail(h, PF_ERR_HIP, std::string("diffuse: ") + hipGetErrorString(e));
+    it += did;
   }
   tables_current(h, s);
   return PF_OK;
@@ -838,6 +881,11 @@ int pf_create(const pf_desc *desc, pf_handle **out) {
   if (const char *e = std::getenv("PFAMD_DIFF_VEC")) h->diff_vec = std::atoi(e) != 0;
   if (const char *e = std::getenv("PFAMD_DIFF_MARCH")) h->diff_march = std::atoi(e) != 0;
   if (const char *e = std::getenv("PFAMD_DIFF_DIRECT")) h->diff_direct = std::atoi(e) != 0;
+  if (const char *e = std::getenv("PFAMD_DIFF_TILE"))
+    // "bx,by,steps" pins the tile, an empty text leaves the rule, anything else switches it off
+    h->diff_tile = !*e || (std::sscanf(e, "%d,%d,%d", &h->tile_pin[0], &h->tile_pin[1],
+                                       &h->tile_pin[2]) == 3 &&
+                           std::min({h->tile_pin[0], h->tile_pin[1], h->tile_pin[2]}) > 0);
   if (const char *e = std::getenv("PFAMD_SWEEP_SPLIT")) h->sweep_split = std::atoi(e) != 0;
   if (const char *e = std::getenv("PFAMD_SWEEP_ROWS")) h->sweep_rows = std::atoi(e);
   if (const char *e = std::getenv("PFAMD_SWEEP_QUEUE")) h->sweep_queue = std::atoi(e) != 0;

@@ -79,3 +79,19 @@ def test_one_launch_substep_bitwise(shape, bc, P, form, params):
     check(shape, bc, P, form, sparse_state(rng, *shape, P), params, (1, 4))
     ids, val, phase, conc = helpers.random_state(rng, *shape, 4, nphase=P)
     check(shape, bc, P, form, (ids, val, phase, conc), params, (3,))
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("shape,P,pin", [((64, 48, 1), 2, ""), ((61, 47, 1), 2, "20,18,12"),
+                                         ((61, 47, 1), 3, "16,16,12"), ((130, 9, 1), 2, "16,16,5"),
+                                         ((5, 4, 1), 2, "16,16,12"), ((2, 3, 1), 3, ""),
+                                         ((40, 1, 13), 2, "16,16,4"), ((400, 30, 1), 2, "")])
+def test_many_substeps_per_launch_bitwise(shape, P, pin, form, params, monkeypatch):
+    """Tiles whose halo is narrower and wider than the domain, partial last tiles, sub-step counts that
+    do not divide, tiles that are nearly all bulk and tiles with more listed cells than entries."""
+    print(f"[gpu] tiles {shape} P={P} pin={pin} form={form}", flush=True)
+    monkeypatch.setenv("PFAMD_DIFF_TILE", pin)
+    rng = np.random.default_rng(12)
+    check(shape, 0, P, form, sparse_state(rng, *shape, P), params, (1, 25))
+    ids, val, phase, conc = helpers.random_state(rng, *shape, 4, nphase=P)
+    check(shape, 0, P, form, (ids, val, phase, conc), params, (13,))
