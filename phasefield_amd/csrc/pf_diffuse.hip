@@ -388,7 +388,7 @@ hipError_t launch_classify(hipStream_t st, const T *pfrac, uint8_t *unit, uint8_
   const unsigned nb = unsigned((ncell + 255) / 256);
   if (unit_ready)  // the bytes are current: only the counters to clear
     hipLaunchKernelGGL(zero_counts_kernel, dim3(1), dim3(64), 0, st, count);
-  else if (nx % 4 == 0)
+  else if (nx % 4 == 0 && reinterpret_cast<uintptr_t>(pfrac) % 16 == 0)
     hipLaunchKernelGGL((unit_phase4_kernel<T, P>), dim3((nb + 3) / 4), dim3(256), 0, st, pfrac,
                        ncell, mask, unit, count);
   else

@@ -85,7 +85,10 @@ hipError_t launch_direct(hipStream_t stream, const typename F::C *cin, typename 
     else if (nx % 2 == 0) go(integral_constant<int, 2>(), integral_constant<int, 2>());
     else go(integral_constant<int, 1>(), integral_constant<int, 1>());
   } else {
-    if (nx % 2 == 0) go(integral_constant<int, 2>(), integral_constant<int, 2>());
+    // (a caller's own array, in the accelerator calls, may be aligned to one value only)
+    const bool aligned =
+        (reinterpret_cast<uintptr_t>(cin) | reinterpret_cast<uintptr_t>(cout)) % 16 == 0;
+    if (nx % 2 == 0 && aligned) go(integral_constant<int, 2>(), integral_constant<int, 2>());
     else go(integral_constant<int, 1>(), integral_constant<int, 2>());
   }
   return hipGetLastError();

@@ -2,16 +2,19 @@
 // pf_gpu_diffusion_solver (GPU_Diffusion_solver, gpu_solver.cpp:204-218) for callers that cannot
 // allocate device memory (code under HIP graph capture, serving loops, harnesses that forbid
 // hipMalloc).  The caller passes value_phase and total_conc in device memory and a stream; the
-// sub-steps run asynchronously on that stream with the LDS-tiled full-formula kernel
-// (diffuse_kernel, bitwise equal to the bulk + listed path of the handle API).
+// sub-steps run asynchronously on that stream with the kernels of the handle API: the bulk flags and
+// the list once per call, then the tile kernel (one plane, several sub-steps per launch) or the
+// one-launch sub-step (3D).  Before, every sub-step ran the full formula for every cell: 256^2 1.19 ms
+// a call of 200 sub-steps, 128^3 8.5 ms.
 //
-// Jacobi sub-steps need a second concentration buffer.  It is `scratch`, a file-scope device array
-// of kNoAllocMaxCells doubles (16 MiB), which every GPU the library is loaded on holds until the
-// process ends.  Host code never passes the array's name to a kernel: its device address is looked
-// up once per device with hipGetSymbolAddress (with that device current) and kept per device.  No
-// part of the buffer needs clearing: the first sub-step writes every cell of it before any read.
-// Calls on one GPU share the buffer, so calls whose work overlaps on one GPU (two streams, two
-// threads) race; calls ordered on one stream do not.
+// What a call needs besides the caller's arrays is in file-scope device arrays with room for
+// kNoAllocMaxCells cells (28.5 MiB), which every GPU the library is loaded on holds until the process
+// ends: Jacobi sub-steps' second concentration buffer (16 MiB), the list of the cells that need the
+// full formula (8 MiB), unit-phase bytes, flags and packed flags (4.5 MiB).  Host code never passes an
+// array's name to a kernel: the device addresses are looked up once per device with
+// hipGetSymbolAddress (with that device current) and kept per device.  No part needs clearing: every
+// pass writes what the next one reads.  Calls on one GPU share the arrays, so calls whose work
+// overlaps on one GPU (two streams, two threads) race; calls ordered on one stream do not.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -20,32 +23,62 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <type_traits>
 
 #include "../../include/phasefield_amd.h"
+#include "pf_diffuse_direct.h"
+#include "pf_diffuse_tile.h"
 #include "pf_handle_access.h"
-#include "pf_kernels.h"
 
 using namespace pfamd;
 
 namespace {
 
 constexpr long kNoAllocMaxCells = 1L << 21;  // 2,097,152 cells (e.g. 128^3)
+constexpr long kMaxListBlocks = kNoAllocMaxCells / (256L * kListChunk);
 __device__ __align__(256) double scratch[kNoAllocMaxCells];
+__device__ __align__(256) int cell_list[kNoAllocMaxCells];
+__device__ __align__(256) uint8_t unit_bytes[kNoAllocMaxCells];
+__device__ __align__(256) uint8_t flag_bytes[kNoAllocMaxCells];
+__device__ __align__(256) uint32_t packed_flags[kNoAllocMaxCells / 16];
+__device__ __align__(256) int list_offsets[kMaxListBlocks + 1];
+__device__ unsigned phase_counts[4];
+
+struct Buffers {
+  double *conc;
+  int *list, *offsets;
+  uint8_t *unit, *flag;
+  uint32_t *packed;
+  unsigned *count;
+};
 
 constexpr int kMaxDevices = 64;
-std::mutex g_scratch_mutex;
-std::array<double *, kMaxDevices> g_scratch_ptr{};
+std::mutex g_buffers_mutex;
+std::array<Buffers, kMaxDevices> g_buffers{};
 
-// device address of `scratch` on the current device (looked up on the first call there)
-hipError_t scratch_on(int dev, double **out) {
-  std::lock_guard<std::mutex> lock(g_scratch_mutex);
-  if (!g_scratch_ptr[dev]) {
-    void *p = nullptr;
-    const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
+// device addresses of the arrays on the current device (looked up on the first call there)
+hipError_t buffers_on(int dev, Buffers *out) {
+  std::lock_guard<std::mutex> lock(g_buffers_mutex);
+  Buffers &b = g_buffers[dev];
+  if (!b.conc) {
+    Buffers n{};
+    auto get = [](auto *&ptr, const void *symbol) {
+      void *p = nullptr;
+      const hipError_t e = hipGetSymbolAddress(&p, symbol);
+      ptr = static_cast<std::remove_reference_t<decltype(ptr)>>(p);
+      return e;
+    };
+    hipError_t e = get(n.list, HIP_SYMBOL(cell_list));
+    if (e == hipSuccess) e = get(n.offsets, HIP_SYMBOL(list_offsets));
+    if (e == hipSuccess) e = get(n.unit, HIP_SYMBOL(unit_bytes));
+    if (e == hipSuccess) e = get(n.flag, HIP_SYMBOL(flag_bytes));
+    if (e == hipSuccess) e = get(n.packed, HIP_SYMBOL(packed_flags));
+    if (e == hipSuccess) e = get(n.count, HIP_SYMBOL(phase_counts));
+    if (e == hipSuccess) e = get(n.conc, HIP_SYMBOL(scratch));
     if (e != hipSuccess) return e;
-    g_scratch_ptr[dev] = static_cast<double *>(p);
+    b = n;
   }
-  *out = g_scratch_ptr[dev];
+  *out = b;
   return hipSuccess;
 }
 
@@ -80,8 +113,8 @@ extern "C" int pf_gpu_diffusion_solver_noalloc(const double *hdiffusivity,
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess || dev < 0 || dev >= kMaxDevices)
     return set_global_error(PF_ERR_NODEVICE, "pf_gpu_diffusion_solver_noalloc: no current device");
-  double *buf = nullptr;
-  if ((e = scratch_on(dev, &buf)) != hipSuccess)
+  Buffers buf;
+  if ((e = buffers_on(dev, &buf)) != hipSuccess)
     return set_global_error(PF_ERR_HIP, std::string("pf_gpu_diffusion_solver_noalloc: "
                                                     "hipGetSymbolAddress: ") +
                                             hipGetErrorString(e));
@@ -102,25 +135,45 @@ extern "C" int pf_gpu_diffusion_solver_noalloc(const double *hdiffusivity,
     dc.D[i] = hdiffusivity[i];
   }
   dc.r = dt / num_loop / (dx * dx);
-  // tile geometry of the LDS kernel: 64 x kDiffTY columns, z split into chunks of >= 16 planes
-  // until about 2048 workgroups (six faces always, as Diff3D sums them, gpu_solver.cpp:160-188)
-  const int tiles_x = (x + 63) / 64, tiles_y = (y + kDiffTY - 1) / kDiffTY;
-  const long tiles = long(tiles_x) * tiles_y;
-  const long nzc = std::max(1L, std::min<long>(z, (2048 + tiles - 1) / tiles));
-  int zc = int((z + nzc - 1) / nzc);
-  zc = std::max(zc, std::min(z, 16));
-  const long nblocks = tiles * ((z + zc - 1) / zc);
-  if (nblocks > 0x7fffffffL)
-    return set_global_error(PF_ERR_INVALID, "pf_gpu_diffusion_solver_noalloc: grid too large");
   const double *pf = dvalue_phase;
-  double *a = dtotal_conc, *b = buf;
-  for (int it = 0; it < num_loop; ++it) {
-    hipLaunchKernelGGL((diffuse_kernel<FormF64, 3, 6, false, kDiffTY>), dim3(unsigned(nblocks)),
-                       dim3(64, kDiffTY + 3), 0, s, a, b, pf, dc, x, y, z, zc, tiles_x, tiles_y,
-                       int(nblocks));
-    std::swap(a, b);
+  double *a = dtotal_conc, *b = buf.conc;
+  // phases whose bulk cells take the reduced form: identity partition
+  unsigned mask = 0;
+  for (int p = 0; p < 3; ++p)
+    if (dc.pk[p][p] == 1.0 && dc.pc[p][p] == 0.0) mask |= 1u << (p + 1);
+  // six faces always, as Diff3D sums them (gpu_solver.cpp:160-188)
+  e = launch_classify<double, 3, 6, false>(s, pf, buf.unit, buf.flag, x, y, z, N, mask, buf.count);
+  if (e != hipSuccess)
+    return set_global_error(PF_ERR_HIP, std::string("pf_gpu_diffusion_solver_noalloc: launch: ") +
+                                            hipGetErrorString(e));
+  TileGeom tile;
+  if (z == 1 && tile_geometry(x, y, 1, num_loop, nullptr, tile)) {
+    for (int left = num_loop; left > 0; left -= tile.steps) {
+      (void)tile_geometry(x, y, 1, left, nullptr, tile);
+      // (the z faces of a one-cell-thick domain carry no flux)
+      hipLaunchKernelGGL((diffuse_tile_kernel<FormF64, 3>), dim3(unsigned(tile.nblocks)),
+                         dim3(kTileNT), 0, s, a, b, pf, buf.flag, dc, tile, N, 0u, 0);
+      std::swap(a, b);
+    }
+  } else {
+    const unsigned nl = unsigned((N + 256L * kListChunk - 1) / (256L * kListChunk));
+    hipLaunchKernelGGL(general_count_kernel, dim3(nl), dim3(256), 0, s, buf.flag,
+                       static_cast<const unsigned *>(nullptr), N, buf.offsets, ListOrder{},
+                       static_cast<int *>(nullptr), buf.packed);
+    hipLaunchKernelGGL(general_scan_kernel, dim3(1), dim3(1024), 0, s, buf.offsets, int(nl),
+                       static_cast<int *>(nullptr));
+    hipLaunchKernelGGL(general_scatter_kernel, dim3(nl), dim3(256), 0, s, buf.flag,
+                       static_cast<const unsigned *>(nullptr), N, buf.offsets, buf.list, ListOrder{});
+    for (int it = 0; it < num_loop && e == hipSuccess; ++it) {
+      e = launch_direct<FormF64, 3, false>(s, a, b, pf, buf.packed, buf.list, buf.offsets + nl, dc, x,
+                                           y, z, (it & 1) != 0);
+      std::swap(a, b);
+    }
+    if (e != hipSuccess)
+      return set_global_error(PF_ERR_HIP, std::string("pf_gpu_diffusion_solver_noalloc: launch: ") +
+                                              hipGetErrorString(e));
   }
-  if (a != dtotal_conc)  // an odd count leaves the result in the scratch buffer
+  if (a != dtotal_conc)  // an odd number of launches leaves the result in the scratch buffer
     hipLaunchKernelGGL(copy_conc_kernel, dim3(unsigned((N + 255) / 256)), dim3(256), 0, s, a,
                        dtotal_conc, N);
   if ((e = hipGetLastError()) != hipSuccess)

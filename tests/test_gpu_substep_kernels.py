@@ -95,3 +95,38 @@ def test_many_substeps_per_launch_bitwise(shape, P, pin, form, params, monkeypat
     check(shape, 0, P, form, sparse_state(rng, *shape, P), params, (1, 25))
     ids, val, phase, conc = helpers.random_state(rng, *shape, 4, nphase=P)
     check(shape, 0, P, form, (ids, val, phase, conc), params, (13,))
+
+
+@pytest.mark.parametrize("skip", [0, 1])
+@pytest.mark.parametrize("shape", [(64, 33, 1), (5, 7, 1), (37, 20, 11), (64, 12, 16), (2, 2, 2)])
+def test_noalloc_kernels_bitwise(shape, skip, params):
+    """The allocation-free call on its tile and one-launch kernels, on arrays that are aligned to 16
+    bytes and to one value only, twice in a row, against the call on host buffers."""
+    import ctypes
+
+    import torch
+
+    from phasefield_amd import gpu_cleanup, gpu_diffusion_solver, lib
+    print(f"[gpu] noalloc kernels {shape} skip={skip}", flush=True)
+    rng = np.random.default_rng(13)
+    n = int(np.prod(shape))
+    D = np.array([params.diffusivity[0][i] for i in range(3)])
+    pk = np.array([[params.part_k[0][i][j] for j in range(3)] for i in range(3)]).T.reshape(-1).copy()
+    pc = np.array([[params.part_c[0][i][j] for j in range(3)] for i in range(3)]).T.reshape(-1).copy()
+    ptr = [a.ctypes.data_as(ctypes.POINTER(ctypes.c_double)) for a in (D, pk, pc)]
+    dt = 0.11 * params.pfm_dt
+    for state in (sparse_state(rng, *shape, 2), helpers.random_state(rng, *shape, 4)):
+        phase, conc = state[2], state[3]
+        dphase = torch.zeros(3 * n + skip, dtype=torch.float64, device="cuda:0")[skip:]
+        dconc = torch.zeros(n + skip, dtype=torch.float64, device="cuda:0")[skip:]
+        dphase.copy_(torch.from_numpy(phase))
+        dconc.copy_(torch.from_numpy(conc))
+        ref = conc.copy()
+        for _ in range(2):
+            gpu_diffusion_solver(D, pk, pc, phase, ref, *shape, dt, params.dx)
+            rc = lib().pf_gpu_diffusion_solver_noalloc(*ptr, dphase.data_ptr(), dconc.data_ptr(), *shape,
+                                                       dt, params.dx,
+                                                       torch.cuda.current_stream().cuda_stream)
+            assert rc == 0, lib().pf_last_error(None)
+        assert np.array_equal(dconc.cpu().numpy(), ref)
+    gpu_cleanup()
