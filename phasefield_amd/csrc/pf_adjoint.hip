@@ -30,6 +30,7 @@
 #include <vector>
 
 #include "../../include/phasefield_amd.h"
+#include "pf_diffuse_direct_impl.h"
 #include "pf_handle_access.h"
 #include "pf_kernels.h"
 
@@ -206,6 +207,27 @@ __global__ __launch_bounds__(256) void adj_general_kernel(
   for (int k = blockIdx.x * 256 + threadIdx.x; k < n; k += gridDim.x * 256)
     dD0 += adj_cell<P, NF, NOFLUX>(list[k], c, pf, lam_in, lam_out, lam_pf, dc, nx, ny, nz);
   block_accumulate(dD0, accD);
+}
+
+// The reverse sub-step in one launch, where the forward one is (pf_diffuse_direct.hip): the listed cells by
+// the first workgroups, the bulk cells of phases other than 1 by the others, the same update with lam
+// for c.  128^3, per reverse sub-step: marching kernel and listed pass 23.7 us, one launch 15.4 us.
+template <int P, bool NOFLUX, int V, int U>
+__global__ __launch_bounds__(256) void adj_direct_kernel(
+    const double *__restrict__ c, const double *__restrict__ pf, const uint32_t *__restrict__ packed,
+    const int *__restrict__ list, const int *__restrict__ count, const double *__restrict__ lam_in,
+    double *__restrict__ lam_out, double *__restrict__ lam_pf, double *__restrict__ accD,
+    const DiffConsts<double> dc, const DirectGeom geo) {
+  const int b = blockIdx.x;
+  if (b < geo.nlist) {
+    const int n = *count;
+    double dD0 = 0.0;
+    for (int k = b * 256 + threadIdx.x; k < n; k += geo.nlist * 256)
+      dD0 += adj_cell<P, 6, NOFLUX>(list[k], c, pf, lam_in, lam_out, lam_pf, dc, geo.nx, geo.ny, geo.nz);
+    block_accumulate(dD0, accD);
+    return;
+  }
+  direct_bulk<FormF64, P, NOFLUX, V, U>(lam_in, lam_out, packed, dc, geo, b - geo.nlist);
 }
 
 // bulk flags of phase 1 -> 0, so those cells join the listed pass
@@ -504,16 +526,15 @@ struct DevState {  // one FP64 state on the device
   double *phi = nullptr, *pf = nullptr, *c = nullptr;
 };
 
-// the device allocations of one adjoint run, released together
+// The device memory of one adjoint run, cut from one block: a first pass over the layout (base null)
+// adds up the sizes, a second hands out the pieces.
 struct Arena {
-  std::vector<void *> ptrs;
-  hipError_t err = hipSuccess;
+  char *base = nullptr;
+  size_t used = 0;
   template <class T> T *get(size_t count) {
-    void *q = nullptr;
-    if (err == hipSuccess) err = hipMalloc(&q, std::max<size_t>(count, 1) * sizeof(T));
-    if (err != hipSuccess) return nullptr;
-    ptrs.push_back(q);
-    return static_cast<T *>(q);
+    T *p = base ? reinterpret_cast<T *>(base + used) : nullptr;
+    used += (std::max<size_t>(count, 1) * sizeof(T) + 255) / 256 * 256;
+    return p;
   }
   DevState state(long N, int KI, int K, int P) {
     DevState d;
@@ -523,10 +544,11 @@ struct Arena {
     d.c = get<double>(size_t(N));
     return d;
   }
-  ~Arena() {
-    for (void *q : ptrs) hipFree(q);
-  }
 };
+// A block of at most this many bytes stays with the handle between runs.  Allocating and freeing it each
+// run took 10 of 43 ms (128^3, 3 steps: 8.5 GB), and freed memory is cleared before it is handed out
+// again, which stalled runs in quick succession to 220 ms and some to seconds.
+constexpr size_t kKeptBlock = size_t(16) << 30;
 
 // Workgroup layout of the bulk sub-step kernels (64 lanes x 4 rows, `cols` x cells per tile row,
 // z split into chunks of at least 8 planes until ~32768 workgroups), as the forward step uses.
@@ -578,51 +600,84 @@ template <int K, int P, int NF, bool NOF> struct Adj {
     const unsigned gb = unsigned((N + 255) / 256), gs = unsigned((N + kAdjBS - 1) / kAdjBS);
     const size_t n8 = size_t(N) * 8;
 
-    Arena ar;
-    std::vector<DevState> ckpt;
-    for (int q = 0; q < nseg; ++q) ckpt.push_back(ar.state(N, KI, K, P));
-    const DevState fin = ar.state(N, KI, K, P);
-    double *lam_c = ar.get<double>(N), *lam_c2 = ar.get<double>(N);
-    double *lam_pf = ar.get<double>(size_t(N) * P), *lam_pf2 = ar.get<double>(size_t(N) * P);
-    double *lam_phi = ar.get<double>(size_t(N) * K), *lam_phi2 = ar.get<double>(size_t(N) * K);
-    double *v2_lam = ar.get<double>(size_t(N) * kStencilMax);
-    uint32_t *v2_id = ar.get<uint32_t>(size_t(N) * kStencilMax);
-    uint8_t *v2_n = ar.get<uint8_t>(N);
-    double *accD = ar.get<double>(gb), *accMS = ar.get<double>(size_t(gs) * 2);
-    double *part = ar.get<double>(gb);
-    double *target = sp->target_conc ? ar.get<double>(N) : nullptr;
+    std::vector<DevState> ckpt(nseg);
+    DevState fin;
+    double *lam_c, *lam_c2, *lam_pf, *lam_pf2, *lam_phi, *lam_phi2, *v2_lam, *accD, *accMS, *part;
+    double *target = nullptr;
+    uint32_t *v2_id, *packed = nullptr;
+    uint8_t *v2_n, *unit_tmp;  // unit_tmp: scratch of the bulk classification
+    int *alist = nullptr, *ablock = nullptr;
     // split reverse sub-step: bulk cells by the forward bulk kernel on lambda, listed cells apart
     const char *env_split = std::getenv("PFAMD_ADJ_SPLIT");
     const bool split = !(env_split && std::strcmp(env_split, "0") == 0);
+    const bool direct = NF == 6 && split && handle_use_direct(h);
     const bool vec = v.nx % 2 == 0;
     const unsigned nl = unsigned((N + 256L * kListChunk - 1) / (256L * kListChunk));
     const unsigned ngen = std::min<unsigned>(gb, 2048);
-    uint8_t *unit_tmp = ar.get<uint8_t>(N);  // scratch of the bulk classification
-    int *alist = split ? ar.get<int>(N) : nullptr;
-    int *ablock = split ? ar.get<int>(nl + 1) : nullptr;
     const TileGeom gvec = tile_geom(v.nx, v.ny, v.nz, NF, 128);
     const TileGeom gsc = tile_geom(v.nx, v.ny, v.nz, NF, 64);
     std::vector<StepData> seg(CK);
-    for (auto &sd : seg) sd.in = ar.state(N, KI, K, P);
+    auto layout = [&](Arena &ar, int nstore) {
+      for (DevState &q : ckpt) q = ar.state(N, KI, K, P);
+      fin = ar.state(N, KI, K, P);
+      lam_c = ar.get<double>(N);
+      lam_c2 = ar.get<double>(N);
+      lam_pf = ar.get<double>(size_t(N) * P);
+      lam_pf2 = ar.get<double>(size_t(N) * P);
+      lam_phi = ar.get<double>(size_t(N) * K);
+      lam_phi2 = ar.get<double>(size_t(N) * K);
+      v2_lam = ar.get<double>(size_t(N) * kStencilMax);
+      v2_id = ar.get<uint32_t>(size_t(N) * kStencilMax);
+      v2_n = ar.get<uint8_t>(N);
+      accD = ar.get<double>(gb);
+      accMS = ar.get<double>(size_t(gs) * 2);
+      part = ar.get<double>(gb);
+      if (sp->target_conc) target = ar.get<double>(N);
+      unit_tmp = ar.get<uint8_t>(N);
+      if (split) {
+        alist = ar.get<int>(N);
+        ablock = ar.get<int>(nl + 1);
+      }
+      if (direct) packed = ar.get<uint32_t>((N + 15) / 16);
+      for (auto &sd : seg) sd.in = ar.state(N, KI, K, P);
+      for (int q = 0; q < nstore; ++q) {
+        seg[q].pf_new = ar.get<double>(size_t(N) * P);
+        seg[q].flag = ar.get<uint8_t>(N);
+        seg[q].count = ar.get<unsigned>(4);
+        seg[q].csub = ar.get<double>(size_t(N) * (nsub + 1));
+      }
+    };
     // Sub-step concentrations for a whole segment when they fit (every step is then recomputed
     // once in the reverse sweep), else for one step (steps are recomputed from the segment's
     // checkpoint to collect their inputs, then once more each).
     const size_t per_step = n8 * (nsub + 1) + n8 * P + size_t(N);
+    Arena fixed;
+    layout(fixed, 0);
     size_t mem_free = 0, mem_total = 0;
-    if (ar.err == hipSuccess) ar.err = hipMemGetInfo(&mem_free, &mem_total);
+    const hipError_t mem_err = hipMemGetInfo(&mem_free, &mem_total);
+    if (mem_err != hipSuccess)
+      return handle_fail(h, PF_ERR_HIP, std::string("adjoint: ") + hipGetErrorString(mem_err));
+    const double left = double(mem_free) + double(handle_adjoint_kept(h)) - double(fixed.used);
     const char *env = std::getenv("PFAMD_ADJ_RECOMPUTE");
     const bool force_step = env && std::strcmp(env, "step") == 0;
-    const bool store_segment = !force_step && double(per_step) * CK < 0.8 * double(mem_free);
+    const bool store_segment = !force_step && double(per_step) * CK < 0.8 * left;
     const int nstore = store_segment ? CK : 1;
-    for (int q = 0; q < nstore; ++q) {
-      seg[q].pf_new = ar.get<double>(size_t(N) * P);
-      seg[q].flag = ar.get<uint8_t>(N);
-      seg[q].count = ar.get<unsigned>(4);
-      seg[q].csub = ar.get<double>(size_t(N) * (nsub + 1));
+    Arena ar;
+    layout(ar, nstore);
+    const size_t bytes = ar.used;
+    ar = Arena{};
+    ar.base = static_cast<char *>(handle_adjoint_block(h, bytes));
+    if (!ar.base) {
+      (void)hipGetLastError();
+      return handle_fail(h, PF_ERR_OOM, "adjoint buffers: out of memory");
     }
-    if (ar.err != hipSuccess)
-      return handle_fail(h, PF_ERR_OOM,
-                         std::string("adjoint buffers: ") + hipGetErrorString(ar.err));
+    layout(ar, nstore);
+    struct Release {  // large blocks go back after the run
+      pf_handle *h;
+      ~Release() {
+        if (handle_adjoint_kept(h) > kKeptBlock) handle_adjoint_release(h);
+      }
+    } release{h};
 
     // first error of the asynchronous copies and clears below (reported by launch_ok)
     hipError_t async_err = hipSuccess;
@@ -729,11 +784,10 @@ template <int K, int P, int NF, bool NOF> struct Adj {
       if (split) {
         // the listed cells of this step: interface cells and bulk cells of phase 1, and, when the
         // plane-marching kernel (one bulk phase for every cell) runs, every cell not of its phase
-        const unsigned *keep = vec && mby ? sd.count : nullptr;
+        const unsigned *keep = vec && mby && !direct ? sd.count : nullptr;
         hipLaunchKernelGGL(adj_list_flag_kernel, dim3(gb), dim3(256), 0, st, sd.flag, N);
         hipLaunchKernelGGL(general_count_kernel, dim3(nl), dim3(256), 0, st, sd.flag, keep, N,
-                           ablock, ListOrder{}, static_cast<int *>(nullptr),
-                           static_cast<uint32_t *>(nullptr));
+                           ablock, ListOrder{}, static_cast<int *>(nullptr), packed);
         hipLaunchKernelGGL(general_scan_kernel, dim3(1), dim3(1024), 0, st, ablock, int(nl),
                            static_cast<int *>(nullptr));
         hipLaunchKernelGGL(general_scatter_kernel, dim3(nl), dim3(256), 0, st, sd.flag, keep, N,
@@ -742,7 +796,20 @@ template <int K, int P, int NF, bool NOF> struct Adj {
       const int mtx = (v.nx + 127) / 128, mty = mby ? (v.ny + mby - 1) / mby : 0;
       const long mnb = mby ? long(mtx) * mty * ((v.nz + mzc - 1) / mzc) : 0;
       for (int s = nsub - 1; s >= 0; --s) {
-        if (split) {
+        if (direct) {
+          if constexpr (NF == 6) {
+            DirectGeom g = direct_geometry(v.nx, v.ny, v.nz, (s & 1) != 0);
+            auto go = [&](auto run) {
+              constexpr int V = decltype(run)::value;
+              set_runs(g, false, V, 2);
+              hipLaunchKernelGGL((adj_direct_kernel<P, NOF, V, 2>), dim3(unsigned(g.nlist + g.nbulk)),
+                                 dim3(256), 0, st, sd.csub + size_t(N) * s, sd.pf_new, packed, alist,
+                                 ablock + nl, lam_c, lam_c2, lam_pf, accD, dc, g);
+            };
+            if (vec) go(std::integral_constant<int, 2>());
+            else go(std::integral_constant<int, 1>());
+          }
+        } else if (split) {
           if (vec && mby == 8)
             hipLaunchKernelGGL((diffuse_bulk_march_kernel<FormF64, P, NF, NOF, 8, 2, 1>),
                                dim3(mnb), dim3(64, 8), 0, st, lam_c, lam_c2, sd.count, dc, v.nx,

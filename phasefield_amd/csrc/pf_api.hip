@@ -111,6 +111,8 @@ struct pf_handle {
   // next sub-step of solute s mixes two tables: 1 = the cells the last sweep copied keep the
   // previous ones, 2 = every cell does (no sweep since the change)
   int retable[PF_MAX_SOLUTE] = {0, 0};
+  void *adj_block = nullptr;  // the adjoint's device memory (handle_adjoint_block)
+  size_t adj_bytes = 0;
   // asynchronous VTI dump: device fields -> pinned host copy (dump stream) -> writer thread
   void *dump_dev = nullptr;      // korn [N] int32, conc [N] float
   void *dump_host = nullptr;     // pinned copy of dump_dev
@@ -805,6 +807,7 @@ void free_all(pf_handle *h) {
   if (h->olist) hipFree(h->olist);
   if (h->gblock) hipFree(h->gblock);
   if (h->packed) hipFree(h->packed);
+  if (h->adj_block) hipFree(h->adj_block);
   if (h->red) hipFree(h->red);
   for (int k = 0; k < 3; ++k)
     for (auto &pr : h->ev[k]) {
@@ -1899,6 +1902,23 @@ int handle_diffuse_io(pf_handle *h, const double *cin, double *cout) {
                                         : diffuse_io_p<3>(h, dc, cin, cout);
   if (e != hipSuccess) return fail(h, PF_ERR_HIP, std::string("diffuse: ") + hipGetErrorString(e));
   return PF_OK;
+}
+bool handle_use_direct(const pf_handle *h) { return use_direct(h, h->NF); }
+void handle_adjoint_release(pf_handle *h) {
+  if (h->adj_block) hipFree(h->adj_block);
+  h->adj_block = nullptr;
+  h->adj_bytes = 0;
+}
+size_t handle_adjoint_kept(const pf_handle *h) { return h->adj_bytes; }
+void *handle_adjoint_block(pf_handle *h, size_t bytes) {
+  if (h->adj_bytes >= bytes) return h->adj_block;
+  handle_adjoint_release(h);
+  if (hipMalloc(&h->adj_block, bytes) != hipSuccess) {
+    h->adj_block = nullptr;
+    return nullptr;
+  }
+  h->adj_bytes = bytes;
+  return h->adj_block;
 }
 void handle_state_changed(pf_handle *h) {
   h->flag_valid = false;

@@ -42,6 +42,29 @@ __global__ void diffuse_direct_kernel(const typename F::C *__restrict__ cin,
                                       const int *__restrict__ list, const int *__restrict__ count,
                                       const DiffConsts<typename F::A> dc, const DirectGeom geo);
 
+// the part of the geometry that does not depend on the run length
+inline DirectGeom direct_geometry(int nx, int ny, int nz, bool flip) {
+  const long n = long(nx) * ny * nz;
+  DirectGeom g;
+  g.nx = nx;
+  g.ny = ny;
+  g.nz = nz;
+  g.flip = flip;
+  // the listed part: one entry per thread up to a sixteenth of the cells (a round of entries is a
+  // chain of three memory latencies and the full formula), at least 64 workgroups where the domain
+  // has that many (40 x 24 x 16 with 4 workgroups: 11.0 us, with 60: 4.3)
+  g.nlist = int(std::min<long>(1024, std::max<long>((n + 4095) / 4096, std::min<long>(64, (n + 255) / 256))));
+  return g;
+}
+// runs of V cells times U planes; pairs: byte pairs in storage order instead
+inline void set_runs(DirectGeom &g, bool pairs, int V, int U) {
+  const long n = long(g.nx) * g.ny * g.nz;
+  g.row = FastDiv(uint32_t(pairs ? g.nx : g.nx / V));
+  g.rows = FastDiv(uint32_t(g.ny));
+  const long items = pairs ? (n + 1) / 2 : long(g.nx / V) * g.ny * ((g.nz + U - 1) / U);
+  g.nbulk = int((items + 255) / 256);
+}
+
 // Run length: 16 bytes where the rows hold a whole number of runs, so that every run is aligned and
 // within one row; rows of odd length take single cells (FP64) or byte pairs in storage order (mixed).
 // Two planes per thread: 128^3 10.5 us against 11.2 with one and 10.7 with four (FP64), 224^3 34.0
@@ -54,28 +77,10 @@ hipError_t launch_direct(hipStream_t stream, const typename F::C *cin, typename 
                          const typename F::T *pfrac, const uint32_t *packed, const int *list,
                          const int *count, const DiffConsts<typename F::A> &dc, int nx, int ny, int nz,
                          bool flip) {
-  const long n = long(nx) * ny * nz;
-  DirectGeom g;
-  g.nx = nx;
-  g.ny = ny;
-  g.nz = nz;
-  g.flip = flip;
-  // the listed part: one entry per thread up to a sixteenth of the cells (a round of entries is a
-  // chain of three memory latencies and the full formula), at least 64 workgroups where the domain
-  // has that many (40 x 24 x 16 with 4 workgroups: 11.0 us, with 60: 4.3)
-  g.nlist = int(std::min<long>(1024, std::max<long>((n + 4095) / 4096, std::min<long>(64, (n + 255) / 256))));
+  DirectGeom g = direct_geometry(nx, ny, nz, flip);
   auto go = [&](auto v, auto u) {
     constexpr int V = decltype(v)::value, U = decltype(u)::value;
-    long items;
-    if constexpr (F::kMixed && V == 1) {
-      g.row = FastDiv(uint32_t(nx));
-      items = (n + 1) / 2;
-    } else {
-      g.row = FastDiv(uint32_t(nx / V));
-      items = long(nx / V) * ny * ((nz + U - 1) / U);
-    }
-    g.rows = FastDiv(uint32_t(ny));
-    g.nbulk = int((items + 255) / 256);
+    set_runs(g, F::kMixed && V == 1, V, U);
     hipLaunchKernelGGL((diffuse_direct_kernel<F, P, NOF, V, U>), dim3(unsigned(g.nlist + g.nbulk)),
                        dim3(256), 0, stream, cin, cout, pfrac, packed, list, count, dc, g);
   };

@@ -36,3 +36,11 @@ void handle_march_shape(const pf_handle *h, int *rows, int *zchunk);
 // one FP64 carbon sub-step from cin into cout with the step's own kernel, flags and factor
 // (value_phase and bulk flags of the handle's current state)
 int handle_diffuse_io(pf_handle *h, const double *cin, double *cout);
+// whether this handle's single sub-steps run as one launch of the direct kernel
+bool handle_use_direct(const pf_handle *h);
+// Device memory of the adjoint, kept between runs and freed with the handle: a block of at least
+// `bytes`, the kept one when it is large enough (null: out of memory).
+void *handle_adjoint_block(pf_handle *h, size_t bytes);
+// bytes of the kept block, and giving it back
+size_t handle_adjoint_kept(const pf_handle *h);
+void handle_adjoint_release(pf_handle *h);
