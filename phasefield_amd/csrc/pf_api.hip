@@ -289,6 +289,11 @@ inline float cutoff_below(double cutoff) {
   return f;
 }
 
+// The growth sweep of the setup is split from this size on; below, its eight launches cost more than
+// the dense kernel saves.  Per iteration, dense / split: 102^3 47 / 82 us, 1024 x 1032 22 / 38,
+// 128^3 77 / 83, 160^3 151 / 127, 256^3 558 / 407.
+constexpr long kIsoSplitCells = 3L << 20;
+
 template <class F, int K, int P, int NF, bool NOF, bool ISO>
 hipError_t launch_sweep(pf_handle *h, const PFConsts<typename F::A> &cs) {
   using T = typename F::T;
@@ -298,11 +303,13 @@ hipError_t launch_sweep(pf_handle *h, const PFConsts<typename F::A> &cs) {
   T *phi2 = static_cast<T *>(h->phi[b]);
   const C *c0 = static_cast<const C *>(h->conc[0][h->ccur[0]]);
   // the split form records which cells it copied, which a change of partition tables needs
-  if (!ISO && (h->sweep_split || h->retable[0] || h->retable[1])) {
+  const bool split = ISO ? h->sweep_split && h->N >= kIsoSplitCells
+                         : h->sweep_split || h->retable[0] || h->retable[1];
+  if (split) {
     // copy cells first (written, or skipped when the destination already holds them), then the
     // full update over the list of the others
     const unsigned nb = blocks_for(h->N), nl = list_blocks(h->N);
-    hipLaunchKernelGGL((sweep_classify_kernel<F, K, NF, NOF>), dim3(nb), dim3(256), 0, h->stream,
+    hipLaunchKernelGGL((sweep_classify_kernel<F, K, NF, NOF, ISO>), dim3(nb), dim3(256), 0, h->stream,
                        h->id[a], phi1, h->id[b], phi2, h->sflag, h->sweep_hist ? 1 : 0,
                        h->p.cutoff, cutoff_below(h->p.cutoff), h->d.nx, h->d.ny, h->d.nz, h->N);
     const ListOrder order = sweep_list_order(h);
@@ -310,7 +317,7 @@ hipError_t launch_sweep(pf_handle *h, const PFConsts<typename F::A> &cs) {
                        static_cast<const unsigned *>(nullptr), h->N, h->gblock, order,
                        static_cast<int *>(nullptr), static_cast<uint32_t *>(nullptr));
     hipLaunchKernelGGL(general_scan_kernel, dim3(1), dim3(1024), 0, h->stream, h->gblock, int(nl),
-                       h->list_len);
+                       ISO ? static_cast<int *>(nullptr) : h->list_len);
     hipLaunchKernelGGL(general_scatter_kernel, dim3(nl), dim3(256), 0, h->stream, h->sflag,
                        static_cast<const unsigned *>(nullptr), h->N, h->gblock, h->glist, order);
     // Every workgroup resident at once (the device's CUs times the kernel's occupancy), each
@@ -326,12 +333,12 @@ hipError_t launch_sweep(pf_handle *h, const PFConsts<typename F::A> &cs) {
     // one kernel.
     constexpr int MODE = (K == 4 && !F::kMixed) ? 1 : 0;
     const void *kfn =
-        reinterpret_cast<const void *>(pf_sweep_kernel<F, K, P, NF, NOF, false, true, MODE>);
+        reinterpret_cast<const void *>(pf_sweep_kernel<F, K, P, NF, NOF, ISO, true, MODE>);
     int &per_cu = h->occupancy[kfn];
     if (per_cu == 0) {
       int n = 0;
       if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-              &n, pf_sweep_kernel<F, K, P, NF, NOF, false, true, MODE>, kSweepBS, 0) !=
+              &n, pf_sweep_kernel<F, K, P, NF, NOF, ISO, true, MODE>, kSweepBS, 0) !=
               hipSuccess ||
           n < 1)
         n = 1;
@@ -344,13 +351,13 @@ hipError_t launch_sweep(pf_handle *h, const PFConsts<typename F::A> &cs) {
     if (MODE == 1)  // the overflow count, olist[N]
       hipLaunchKernelGGL(zero_counts_kernel, dim3(1), dim3(64), 0, h->stream,
                          reinterpret_cast<unsigned *>(h->olist + h->N));
-    hipLaunchKernelGGL((pf_sweep_kernel<F, K, P, NF, NOF, false, true, MODE>), dim3(ng),
+    hipLaunchKernelGGL((pf_sweep_kernel<F, K, P, NF, NOF, ISO, true, MODE>), dim3(ng),
                        dim3(kSweepBS), 0, h->stream, h->id[a], phi1, h->id[b], phi2,
                        static_cast<T *>(h->pfrac), c0, cs, h->d.nx, h->d.ny, h->d.nz, h->N, h->glist,
                        h->gblock + nl, h->sweep_queue ? h->squeue : static_cast<int *>(nullptr),
                        h->sflag, h->unit, h->bulk_mask, h->olist);
     if (MODE == 1)
-      hipLaunchKernelGGL((pf_sweep_kernel<F, K, P, NF, NOF, false, true, 2>),
+      hipLaunchKernelGGL((pf_sweep_kernel<F, K, P, NF, NOF, ISO, true, 2>),
                          dim3(unsigned(std::max(h->num_cu, 1))), dim3(kSweepBS), 0, h->stream,
                          h->id[a], phi1, h->id[b], phi2, static_cast<T *>(h->pfrac), c0, cs,
                          h->d.nx, h->d.ny, h->d.nz, h->N, h->olist, h->olist + h->N,
@@ -1510,8 +1517,12 @@ int pf_setup_construct(pf_handle *h, const double *seeds, int G, double reductio
   double *phi = static_cast<double *>(h->phi[0]), *pf = static_cast<double *>(h->pfrac);
   if (e == hipSuccess) {
     h->cur = 0;
+    // blocks of 8 x 8 x 4 cells, 16 x 16 of a plane
+    const long w = h->d.nz == 1 ? 16 : 8, wz = h->d.nz == 1 ? 1 : 4;
+    const long vblocks = std::min<long>((h->d.nx + w - 1) / w * ((h->d.ny + w - 1) / w) *
+                                            ((h->d.nz + wz - 1) / wz), 1L << 20);
 #define PF_VOR(KK, PP)                                                                        \
-  hipLaunchKernelGGL((voronoi_kernel<KK, PP>), dim3(blocks_for(h->N)), dim3(256), 0, h->stream, \
+  hipLaunchKernelGGL((voronoi_kernel<KK, PP>), dim3(unsigned(vblocks)), dim3(256), 0, h->stream, \
                      dseeds, G, reduction, h->d.nx, h->d.ny, h->d.nz, h->N, h->id[0], phi, pf)
     if (K == 4 && P == 2) PF_VOR(4, 2);
     else if (K == 4) PF_VOR(4, 3);
@@ -1523,15 +1534,16 @@ int pf_setup_construct(pf_handle *h, const double *seeds, int G, double reductio
   if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
   hipFree(dseeds);
   if (e != hipSuccess) return fail(h, PF_ERR_HIP, std::string("voronoi: ") + hipGetErrorString(e));
-  // slot-1 buffer must hold zeros where Iso_growth leaves slots unwritten
-  HIPCHK(h, hipMemsetAsync(h->id[1], 0, size_t(h->N) * h->KI * 2, h->stream));
-  HIPCHK(h, hipMemsetAsync(h->phi[1], 0, size_t(h->N) * K * 8, h->stream));
+  h->sweep_hist = false;  // (a new state)
   // Iso_growth iterations with factor 0.5/dims*dx*dx (MicrostructureConstruction.cpp:216)
   PFConsts<double> cs = make_pf_consts<double>(h);
   cs.dt = 0.5 / double(h->dims) * h->p.dx * h->p.dx;
   for (int it = 0; it < n_iso; ++it) {
     hipError_t le = dispatch_sweep<FormF64, true>(h, cs);
-    if (le != hipSuccess) return fail(h, PF_ERR_HIP, std::string("iso: ") + hipGetErrorString(le));
+    if (le != hipSuccess) {
+      h->sweep_hist = false;
+      return fail(h, PF_ERR_HIP, std::string("iso: ") + hipGetErrorString(le));
+    }
   }
   for (int s = 0; s < h->d.nsolute; ++s) {
     h->ccur[s] = 0;
@@ -1593,26 +1605,24 @@ int pf_setup_nucleate(pf_handle *h, int n_nuclei, float radius, const double *nu
   hipSetDevice(h->d.device);
   const int K = h->d.depth, P = h->d.nphase;
   const long N = h->N;
-  float *flag = nullptr, *pv = nullptr;
+  // scratch: the flag, the painted cells, the flag's maximum per chunk and overall
+  const int nchunk = int((N + kFlagChunk - 1) / kFlagChunk);
+  float *flag = nullptr;
   uint8_t *mark = nullptr;
-  long long *pi = nullptr;
-  const int nparts = int(std::min<long>(1024, (N + 4095) / 4096));
-  const long per = (N + nparts - 1) / nparts;
-  const int nb = int((N + per - 1) / per);
+  unsigned long long *best = nullptr;  // then the centre and the paint's count of workgroups
   auto cleanup = [&]() {
     if (flag) hipFree(flag);
     if (mark) hipFree(mark);
-    if (pv) hipFree(pv);
-    if (pi) hipFree(pi);
+    if (best) hipFree(best);
   };
   hipError_t e = hipMalloc(&flag, N * 4);
   if (e == hipSuccess) e = hipMalloc(&mark, N);
-  if (e == hipSuccess) e = hipMalloc(&pv, nparts * 4);
-  if (e == hipSuccess) e = hipMalloc(&pi, nparts * 8);
+  if (e == hipSuccess) e = hipMalloc(&best, (size_t(nchunk) + 1) * 8);
   if (e != hipSuccess) {
     cleanup();
     return fail(h, PF_ERR_OOM, "nucleation scratch allocation failed");
   }
+  int *centre = reinterpret_cast<int *>(best + nchunk);
   const DiffConsts<double> dc = make_diff_consts<double>(h->p, 0, 0.0);
   const uint64_t key = [&] {
     uint64_t z = seed + 0x9E3779B97F4A7C15ULL;
@@ -1633,17 +1643,19 @@ int pf_setup_nucleate(pf_handle *h, int n_nuclei, float radius, const double *nu
   e = hipGetLastError();
   const int R = int(std::ceil(2.0f * radius));
   const int ext[3] = {h->d.nx, h->d.ny, h->d.nz};
-  int cntv[3];
+  int cntv[3];  // the box, whole axes where it does not fit
   for (int d = 0; d < 3; ++d) cntv[d] = (2 * R + 1 >= ext[d]) ? ext[d] : 2 * R + 1;
-  const long box = long(cntv[0]) * cntv[1] * cntv[2];
+  // chunks per plane of the box: two runs, each with a partial chunk at either end
+  const dim3 box(unsigned(long(cntv[1]) * h->d.nx / kFlagChunk + 4), unsigned(std::min(cntv[2], 32768)));
+  if (e == hipSuccess && n_nuclei > 0) {
+    hipLaunchKernelGGL(flag_chunks_kernel, dim3(nchunk), dim3(1024), 0, h->stream, flag, int(N), best);
+    hipLaunchKernelGGL(flag_centre_kernel, dim3(1), dim3(1024), 0, h->stream, best, nchunk, centre);
+  }
   for (int q = 1; q <= n_nuclei && e == hipSuccess; ++q) {
-    hipLaunchKernelGGL(argmax_stage1, dim3(nb), dim3(256), 0, h->stream, flag, N, per, pv, pi);
-    hipLaunchKernelGGL(argmax_stage2, dim3(1), dim3(256), 0, h->stream, pv, pi, nb);
-#define PF_PAINT(KK, PP)                                                                      \
-  hipLaunchKernelGGL((nucleus_paint_kernel<KK, PP>), dim3(blocks_for(box)), dim3(256), 0,      \
-                     h->stream, pi, codes[q], radius, R, h->d.nx, h->d.ny, h->d.nz, cntv[0],  \
-                     cntv[1],                                                                 \
-                     cntv[2], h->id[h->cur], phi, pf, flag, mark)
+#define PF_PAINT(KK, PP)                                                                        \
+  hipLaunchKernelGGL((nucleus_paint_kernel<KK, PP>), box, dim3(1024), 0, h->stream, centre,      \
+                     codes[q], radius, R, h->d.nx, h->d.ny, h->d.nz, cntv[1], cntv[2],           \
+                     h->id[h->cur], phi, pf, flag, mark, int(N), best, nchunk)
     if (K == 4 && P == 2) PF_PAINT(4, 2);
     else if (K == 4) PF_PAINT(4, 3);
     else if (P == 2) PF_PAINT(6, 2);

@@ -28,7 +28,7 @@ __global__ void zero_counts_kernel(unsigned *__restrict__ count);
 __global__ void zero_queue_kernel(int *__restrict__ queue);
 
 // copy cells of the sweep written directly, the others flagged 0 for the listed sweep
-template <class F, int K, int NF, bool NOFLUX>
+template <class F, int K, int NF, bool NOFLUX, bool ISO>
 __global__ void sweep_classify_kernel(const uint16_t *__restrict__ id1,
                                       const typename F::T *__restrict__ phi1,
                                       uint16_t *__restrict__ id2, typename F::T *__restrict__ phi2,
@@ -232,15 +232,18 @@ __global__ void nucleation_flag_kernel(const uint16_t *__restrict__ id,
                                        const double *__restrict__ c0, const DiffConsts<double> dc,
                                        uint64_t seed_key, long ncell, float *__restrict__ flag,
                                        uint8_t *__restrict__ mark);
-__global__ void argmax_stage1(const float *__restrict__ flag, long ncell, long per_block,
-                              float *__restrict__ pv, long long *__restrict__ pi);
-__global__ void argmax_stage2(float *__restrict__ pv, long long *__restrict__ pi, int nparts);
+constexpr int kFlagChunk = 4096;  // cells per kept maximum of the nucleation flag
+__global__ void flag_chunks_kernel(const float *__restrict__ flag, int ncell,
+                                   unsigned long long *__restrict__ best);
+__global__ void flag_centre_kernel(const unsigned long long *__restrict__ best, int nchunk,
+                                   int *__restrict__ centre);
 template <int K, int P>
-__global__ void nucleus_paint_kernel(const long long *__restrict__ center, int code, float radius,
-                                     int R, int nx, int ny, int nz, int cx_n, int cy_n, int cz_n,
+__global__ void nucleus_paint_kernel(int *__restrict__ centre, int code, float radius, int R,
+                                     int nx, int ny, int nz, int cy_n, int cz_n,
                                      uint16_t *__restrict__ id, double *__restrict__ phi,
                                      double *__restrict__ pfrac, float *__restrict__ flag,
-                                     uint8_t *__restrict__ mark);
+                                     uint8_t *__restrict__ mark, int ncell,
+                                     unsigned long long *__restrict__ best, int nchunk);
 template <class F>
 __global__ void vti_fields_kernel(const uint16_t *__restrict__ id, int KI,
                                   const typename F::C *__restrict__ c, long ncell,
