@@ -617,8 +617,8 @@ template <int K, int P, int NF, bool NOF> struct Adj {
     const TileGeom gvec = tile_geom(v.nx, v.ny, v.nz, NF, 128);
     const TileGeom gsc = tile_geom(v.nx, v.ny, v.nz, NF, 64);
     std::vector<StepData> seg(CK);
-    auto layout = [&](Arena &ar, int nstore) {
-      for (DevState &q : ckpt) q = ar.state(N, KI, K, P);
+    auto layout = [&](Arena &ar, int nstore, int nckpt) {
+      for (int q = 0; q < nckpt; ++q) ckpt[q] = ar.state(N, KI, K, P);
       fin = ar.state(N, KI, K, P);
       lam_c = ar.get<double>(N);
       lam_c2 = ar.get<double>(N);
@@ -647,12 +647,14 @@ template <int K, int P, int NF, bool NOF> struct Adj {
         seg[q].csub = ar.get<double>(size_t(N) * (nsub + 1));
       }
     };
-    // Sub-step concentrations for a whole segment when they fit (every step is then recomputed
-    // once in the reverse sweep), else for one step (steps are recomputed from the segment's
-    // checkpoint to collect their inputs, then once more each).
+    // Sub-step concentrations for a whole segment when they fit: the last segment's are kept as the
+    // forward run computes them, every other step is recomputed once in the reverse sweep.  Else for
+    // one step (steps are recomputed from the segment's checkpoint to collect their inputs, then
+    // once more each).  The segments are counted from the end, so that the last one is full.
+    // 128^3, 3 steps, two to a segment: all three recomputed 27.5 ms, the first alone 23.1 ms.
     const size_t per_step = n8 * (nsub + 1) + n8 * P + size_t(N);
     Arena fixed;
-    layout(fixed, 0);
+    layout(fixed, 0, nseg);
     size_t mem_free = 0, mem_total = 0;
     const hipError_t mem_err = hipMemGetInfo(&mem_free, &mem_total);
     if (mem_err != hipSuccess)
@@ -661,9 +663,11 @@ template <int K, int P, int NF, bool NOF> struct Adj {
     const char *env = std::getenv("PFAMD_ADJ_RECOMPUTE");
     const bool force_step = env && std::strcmp(env, "step") == 0;
     const bool store_segment = !force_step && double(per_step) * CK < 0.8 * left;
-    const int nstore = store_segment ? CK : 1;
+    const int nstore = store_segment ? CK : 1, nckpt = store_segment ? nseg - 1 : nseg;
+    const int rec0 = store_segment ? nsteps - CK : nsteps;  // the first step kept as it runs
+    auto seg_begin = [&](int sg) { return std::max(0, nsteps - (nseg - sg) * CK); };
     Arena ar;
-    layout(ar, nstore);
+    layout(ar, nstore, nckpt);
     const size_t bytes = ar.used;
     ar = Arena{};
     ar.base = static_cast<char *>(handle_adjoint_block(h, bytes));
@@ -671,7 +675,7 @@ template <int K, int P, int NF, bool NOF> struct Adj {
       (void)hipGetLastError();
       return handle_fail(h, PF_ERR_OOM, "adjoint buffers: out of memory");
     }
-    layout(ar, nstore);
+    layout(ar, nstore, nckpt);
     struct Release {  // large blocks go back after the run
       pf_handle *h;
       ~Release() {
@@ -716,15 +720,39 @@ template <int K, int P, int NF, bool NOF> struct Adj {
                                                               hipGetErrorString(e));
     };
 
+    // run the step whose input the handle holds and keep its sub-step data in slot q
+    auto record = [&](int q) -> int {
+      StepData &sd = seg[q];
+      int r = pf_phase_field_sweep(h);
+      if (r != PF_OK) return r;
+      const DevState cur = on_handle();
+      async_ok(hipMemcpyAsync(sd.pf_new, cur.pf, n8 * P, hipMemcpyDeviceToDevice, st));
+      (void)launch_classify<double, P, NF, NOF>(st, sd.pf_new, unit_tmp, sd.flag, v.nx, v.ny,
+                                                 v.nz, N, v.bulk_mask, sd.count);
+      async_ok(hipMemcpyAsync(sd.csub, cur.c, n8, hipMemcpyDeviceToDevice, st));
+      for (int s = 0; s < nsub && r == PF_OK; ++s)
+        r = handle_diffuse_io(h, sd.csub + size_t(N) * s, sd.csub + size_t(N) * (s + 1));
+      if (r != PF_OK) return r;
+      // the step's output carbon, the next step's input
+      async_ok(hipMemcpyAsync(cur.c, sd.csub + size_t(N) * nsub, n8, hipMemcpyDeviceToDevice, st));
+      return launch_ok();
+    };
+
     // ---- forward with checkpoints ----
     if (target) async_ok(hipMemcpyAsync(target, sp->target_conc, n8, hipMemcpyHostToDevice, st));
     const auto t0 = std::chrono::steady_clock::now();
     double loss = 0.0;
     std::vector<double> frac(sp->n_samples, 0.0);
     int rc = PF_OK;
-    for (int k = 0; k < nsteps && rc == PF_OK; ++k) {
-      if (k % CK == 0) save(ckpt[k / CK]);
-      rc = pf_step(h, 1);
+    for (int k = 0, sg = 0; k < nsteps && rc == PF_OK; ++k) {
+      if (k >= rec0) {
+        save(seg[k - rec0].in);
+        rc = record(k - rec0);
+        handle_count_substeps(h, nsub);
+      } else {
+        if (k == seg_begin(sg)) save(ckpt[sg++]);
+        rc = pf_step(h, 1);
+      }
       const int q = sample_index(k + 1);
       if (rc == PF_OK && q >= 0) {
         pf_stats s;
@@ -753,23 +781,6 @@ template <int K, int P, int NF, bool NOF> struct Adj {
     const auto t1 = std::chrono::steady_clock::now();
 
     // ---- reverse ----
-    // recompute the step whose input the handle holds into slot q
-    auto recompute = [&](int q) -> int {
-      StepData &sd = seg[q];
-      int r = pf_phase_field_sweep(h);
-      if (r != PF_OK) return r;
-      const DevState cur = on_handle();
-      async_ok(hipMemcpyAsync(sd.pf_new, cur.pf, n8 * P, hipMemcpyDeviceToDevice, st));
-      (void)launch_classify<double, P, NF, NOF>(st, sd.pf_new, unit_tmp, sd.flag, v.nx, v.ny,
-                                                 v.nz, N, v.bulk_mask, sd.count);
-      async_ok(hipMemcpyAsync(sd.csub, cur.c, n8, hipMemcpyDeviceToDevice, st));
-      for (int s = 0; s < nsub && r == PF_OK; ++s)
-        r = handle_diffuse_io(h, sd.csub + size_t(N) * s, sd.csub + size_t(N) * (s + 1));
-      if (r != PF_OK) return r;
-      // the step's output carbon, the next step's input
-      async_ok(hipMemcpyAsync(cur.c, sd.csub + size_t(N) * nsub, n8, hipMemcpyDeviceToDevice, st));
-      return launch_ok();
-    };
     // reverse step k from slot q (sub-step data) and its input state
     auto reverse = [&](int q, int k, const DevState &in) -> int {
       const StepData &sd = seg[q];
@@ -854,22 +865,27 @@ template <int K, int P, int NF, bool NOF> struct Adj {
       return launch_ok();
     };
     for (int sg = nseg - 1; sg >= 0 && rc == PF_OK; --sg) {
-      const int k0 = sg * CK, k1 = std::min(nsteps, k0 + CK);
-      load(ckpt[sg]);
+      const int k0 = seg_begin(sg), k1 = nsteps - (nseg - 1 - sg) * CK;
       if (store_segment) {
-        for (int k = k0; k < k1 && rc == PF_OK; ++k) {
-          save(seg[k - k0].in);
-          rc = recompute(k - k0);
+        // (the input of a recomputed segment's first step is its checkpoint)
+        auto input = [&](int k) -> const DevState & {
+          return k == k0 && k < rec0 ? ckpt[sg] : seg[k - k0].in;
+        };
+        if (k0 < rec0) load(ckpt[sg]);
+        for (int k = k0; k < k1 && k < rec0 && rc == PF_OK; ++k) {
+          if (k > k0) save(seg[k - k0].in);
+          rc = record(k - k0);
         }
-        for (int k = k1 - 1; k >= k0 && rc == PF_OK; --k) rc = reverse(k - k0, k, seg[k - k0].in);
+        for (int k = k1 - 1; k >= k0 && rc == PF_OK; --k) rc = reverse(k - k0, k, input(k));
       } else {
+        load(ckpt[sg]);
         for (int k = k0; k < k1 && rc == PF_OK; ++k) {
           save(seg[k - k0].in);
           if (k + 1 < k1) rc = pf_step(h, 1);
         }
         for (int k = k1 - 1; k >= k0 && rc == PF_OK; --k) {
           load(seg[k - k0].in);
-          rc = recompute(0);
+          rc = record(0);
           if (rc == PF_OK) rc = reverse(0, k, seg[k - k0].in);
         }
       }

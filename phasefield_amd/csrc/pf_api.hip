@@ -1915,6 +1915,7 @@ int handle_diffuse_io(pf_handle *h, const double *cin, double *cout) {
   if (e != hipSuccess) return fail(h, PF_ERR_HIP, std::string("diffuse: ") + hipGetErrorString(e));
   return PF_OK;
 }
+void handle_count_substeps(pf_handle *h, int n) { h->csub[0] += uint32_t(n); }
 bool handle_use_direct(const pf_handle *h) { return use_direct(h, h->NF); }
 void handle_adjoint_release(pf_handle *h) {
   if (h->adj_block) hipFree(h->adj_block);

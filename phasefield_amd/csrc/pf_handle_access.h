@@ -36,6 +36,8 @@ void handle_march_shape(const pf_handle *h, int *rows, int *zchunk);
 // one FP64 carbon sub-step from cin into cout with the step's own kernel, flags and factor
 // (value_phase and bulk flags of the handle's current state)
 int handle_diffuse_io(pf_handle *h, const double *cin, double *cout);
+// n carbon sub-steps done outside of pf_step (the sub-step counter of checkpoints)
+void handle_count_substeps(pf_handle *h, int n);
 // whether this handle's single sub-steps run as one launch of the direct kernel
 bool handle_use_direct(const pf_handle *h);
 // Device memory of the adjoint, kept between runs and freed with the handle: a block of at least

@@ -130,3 +130,38 @@ def test_noalloc_kernels_bitwise(shape, skip, params):
             assert rc == 0, lib().pf_last_error(None)
         assert np.array_equal(dconc.cpu().numpy(), ref)
     gpu_cleanup()
+
+
+@pytest.mark.parametrize("shape,steps,every", [((20, 18, 10), 1, 1), ((20, 18, 10), 3, 2),
+                                               ((33, 9, 7), 5, 3), ((40, 21, 1), 3, 3)])
+def test_adjoint_leaves_the_stepped_state(shape, steps, every, params):
+    """The steps whose sub-steps are kept as they run leave what plain steps leave: the checkpoint
+    (state and sub-step counter) and the step after it; a run that recomputes every step from its
+    checkpoints gives the same gradients."""
+    print(f"[gpu] adjoint state {shape} steps={steps} every={every}", flush=True)
+    nx, ny, nz = shape
+    q = PfParams.from_buffer_copy(params)
+    q.dims = 3 - (nz == 1)
+    q.n_sub[0] = 7
+    state = sparse_state(np.random.default_rng(14), *shape, 2)
+    blob, grad = [], []
+    for mode in ("plain", "segment", "step"):
+        g = Domain(nx, ny, nz, depth=4)
+        g.set_params(q)
+        g.upload(*state)
+        if mode == "plain":
+            g.step(steps)
+        else:
+            with pytest.MonkeyPatch.context() as mp:
+                mp.setenv("PFAMD_ADJ_RECOMPUTE", mode)
+                grad.append(g.adjoint(steps, [steps], [0.3], checkpoint_every=every))
+        a = g.checkpoint()
+        g.step(1)
+        blob.append((a, g.download()["conc"]))
+        g.close()
+    assert blob[0][0] == blob[1][0]
+    for _, conc in blob[1:]:
+        assert np.array_equal(conc, blob[0][1])
+    for key in ("loss", "d_mobility", "d_sigma", "d_diff_gamma"):
+        assert grad[0][key] == grad[1][key], key
+    assert np.array_equal(grad[0]["d_conc0"], grad[1]["d_conc0"])
