@@ -1120,8 +1120,8 @@ __global__ __launch_bounds__(256) void diffuse_general_kernel(
     StencilLoad<F, P, NF> s0, s1;
     stencil_load<F, P, NF>(cin, pfrac, i0, ncell, nb0, s0);
     stencil_load<F, P, NF>(cin, pfrac, i1, ncell, nb1, s1);
-    stencil_update<F, P, NF>(cout, i0, ncell, s0, dc);
-    if (two) stencil_update<F, P, NF>(cout, i1, ncell, s1, dc);
+    stencil_update<F, P, NF, true>(cout, i0, ncell, s0, dc);
+    if (two) stencil_update<F, P, NF, true>(cout, i1, ncell, s1, dc);
   }
 }
 
