@@ -13,7 +13,8 @@ by stream synchronisation.
 Roofline of the dominant kernel, the plane-marching diffusion kernel (about 80 % of a step): the
 bytes it must move per launch (every cell's stored concentration read once and written once: FP64
 8 + 8 B, mixed 4 + 1 B each way) over its mean launch time from HIP event pairs around a sample of
-its launches inside the timed region, on the stream it runs on.  `substep` adds the listed pass
+its launches inside the timed region, on the stream it runs on (domains that do not take it: the same
+bytes over the sub-step, named by its kernel).  `substep` adds the listed pass
 (the cells next to a phase boundary, full formula) with the list length read from the device, and
 the gaps between the two launches.  `model_8d` states the same run in the compulsory-traffic model
 of the scope document (every cell reads value_phase; 24 / 32 B per cell per sub-step).
@@ -123,6 +124,12 @@ def measured_traffic(workload: str) -> dict:
                         rec["stale"] = rec.get("sources") != kernel_source_hash()
                         return rec
     return {}
+
+
+def substep_kernel_name(is_mixed: bool, nphase: int, dims: int) -> str:
+    """The kernel of a sub-step that is not the marching kernel's (2D: several sub-steps a launch)."""
+    kernel = "diffuse_tile_kernel" if dims == 2 else "diffuse_direct_kernel"
+    return f"{kernel}<{'FormMixed' if is_mixed else 'FormF64'}, {nphase}>"
 
 
 def march_kernel_name(mixed: bool, nphase: int, noflux: bool, rows: int) -> str:
@@ -498,12 +505,16 @@ def main() -> int:
         sweep_listed, diff_listed = dom.list_lengths()
         rows, zc = dom.march_shape()
         st = dom.reduce()
-        sub_us = t["sub"][0] / t["sub"][1] * 1e3
-        march_us = t["march"][0] / max(t["march"][1], 1) * 1e3
+        sub_us = t["sub"][0] / max(t["sub"][1], 1) * 1e3
+        # domains whose whole sub-step is one launch (or several sub-steps of a plane) have no
+        # marching launches: the roofline is the sub-step's then
+        dominant = "march" if t["march"][1] else "sub"
+        march_us = t[dominant][0] / max(t[dominant][1], 1) * 1e3
         sweep_us = t["sweep"][0] / t["sweep"][1] * 1e3
         bpc = march_bytes_per_cell(is_mixed)
-        achieved = N * bpc / (march_us * 1e-6) / 1e9
-        kname = march_kernel_name(is_mixed, d.nphase, noflux, rows)
+        achieved = N * bpc / (max(march_us, 1e-3) * 1e-6) / 1e9
+        kname = (march_kernel_name(is_mixed, d.nphase, noflux, rows) if dominant == "march" else
+                 substep_kernel_name(is_mixed, d.nphase, 2 if d.nz == 1 else 3))
         # the summary records each profiled tile shape's bytes by kernel name; the tuner's pick
         # on this device selects one (none when it picked a shape the summary did not profile)
         measured = (traffic.get("march", {}).get(kname)
@@ -518,7 +529,7 @@ def main() -> int:
                          "traffic": measured,
                          "kernel": kname, "tile_rows": rows, "z_chunk": zc,
                          "bytes_per_cell": bpc, "cells_per_launch": N,
-                         "launch_us": round(march_us, 2), "launches_timed": t["march"][1],
+                         "launch_us": round(march_us, 2), "launches_timed": t[dominant][1],
                          "traffic_source": (f"{traffic.get('file')} (kernel sources "
                                             f"{traffic.get('sources')}"
                                             f"{', stale: not used' if traffic.get('stale') else ''})"
@@ -529,12 +540,13 @@ def main() -> int:
                         "listed_cells": diff_listed,
                         "listed_fraction": round(diff_listed / N, 6),
                         "bytes": sub_bytes, "listed_bytes_per_cell": lbpc,
-                        "achieved_gbs": round(sub_bytes / (sub_us * 1e-6) / 1e9, 1),
-                        "frac": round(sub_bytes / (sub_us * 1e-6) / 1e9 / HBM_PEAK_GBS, 4)},
+                        "achieved_gbs": round(sub_bytes / (max(sub_us, 1e-3) * 1e-6) / 1e9, 1),
+                        "frac": round(sub_bytes / (max(sub_us, 1e-3) * 1e-6) / 1e9 / HBM_PEAK_GBS, 4)},
             "sweep": {"us": round(sweep_us, 1), "listed_cells": sweep_listed,
                       "listed_fraction": round(sweep_listed / N, 6)},
         }
-        log(f"{name}: {res[name]['ms_per_step']:.2f} ms/step, march {march_us:.1f} us "
+        log(f"{name}: {res[name]['ms_per_step']:.2f} ms/step, "
+            f"{'march' if dominant == 'march' else 'one launch'} {march_us:.1f} us "
             f"({achieved:.0f} GB/s), sub-step {sub_us:.1f} us ({res[name]['substep']['frac']:.3f} of "
             f"peak, {diff_listed} listed), sweep {sweep_us:.0f} us ({sweep_listed} listed)")
 
@@ -569,7 +581,7 @@ def main() -> int:
                        "dtype": "f64", "roofline": f64["roofline"], "substep": f64["substep"],
                        "sweep": f64["sweep"], "model_8d": f64["model_8d"]}
         out["mixed_over_fp64"] = round(mx["value"] / f64["value"], 4)
-        out["march_fp64_over_mixed"] = round(f64["roofline"]["launch_us"] / mx["roofline"]["launch_us"], 4)
+        out["march_fp64_over_mixed"] = round(f64["roofline"]["launch_us"] / max(mx["roofline"]["launch_us"], 1e-3), 4)
         done = args.warmup + args.steps
         if args.accuracy_steps > done:
             log(f"accuracy: both forms to step {args.accuracy_steps}")

@@ -16,9 +16,11 @@
 //                        local concentration, mobility and interface-energy scales).
 //   adj_gather_kernel    scatter of the neighbour-sum adjoints back to the slots that fed them, as
 //                        a gather over the stencil (a neighbour slot feeds the entry with its id).
-// Schedule: the forward run keeps a device checkpoint every `checkpoint_every` steps; the reverse
-// sweep recomputes each segment, then per step recomputes and stores the sub-step concentrations
-// and runs the reverse kernels backwards.
+//   adj_direct_kernel    the reverse sub-step in one launch, where the forward one is.
+// Schedule: the forward run keeps a device checkpoint every `checkpoint_every` steps, counted from the
+// end, and the sub-step concentrations of the last of these segments; the reverse sweep runs each
+// earlier segment once more from its checkpoint, storing the sub-step concentrations, and runs the
+// reverse kernels backwards.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -17,14 +17,17 @@
 //   diffuse_bulk_vec_kernel    bulk cells only, 16-byte runs per lane, U planes per batch
 //   diffuse_bulk_march_kernel  the bulk update of the most common bulk phase for every cell, no
 //                          per-cell flag read, 16-byte runs per lane, plane-marching with the
-//                          tile's rows in LDS (the default sub-step when nx is a multiple of the
-//                          run length; its tile height and z-chunk are picked by timing)
+//                          tile's rows in LDS (the default sub-step of large 3D domains when nx is
+//                          a multiple of the run length; its tile height and z-chunk are picked by
+//                          timing)
 //   diffuse_general_kernel the full formula over the per-sweep list of the cells the bulk kernels
 //                          leave (non-bulk cells; with the plane-marching kernel, every cell
 //                          whose flag is not its bulk phase)
 //   diffuse_kernel         full formula for every cell, LDS-tiled (selected with
 //                          PFAMD_DIFF_KERNEL=lds; kept as an independent path for the parity tests)
 //   general_count/scan/scatter_kernel  the storage-order list of the cells a bulk kernel leaves
+// Smaller 3D domains and odd rows take one launch per sub-step (pf_diffuse_direct.hip), planes several
+// sub-steps per launch (pf_diffuse_tile.hip).
 //
 // diffuse_kernel layout: a workgroup owns a 64 x TY column tile and marches through a z-chunk, one
 // plane per iteration.  It has TY + 3 wavefronts: TY interior rows, the rows above and below the tile, and
@@ -34,7 +37,8 @@
 // and the interior lanes then apply the 7-point flux.  z neighbours of a column stay in
 // registers; the global loads of a column run two planes ahead of their use.
 // A phase absent from a cell (phi_p == 0) gives zero weight on all its faces, so its partition is
-// not computed; weights sqrt(0) and sqrt(1) are exact and skip the square-root sequence; the weight
+// not used; weights sqrt(0) and sqrt(1) are exact (both are skipped, but for the FP64 listed pass, whose
+// sequences interleave instead); the weight
 // of a z face is shared by the two planes it separates (the product is commutative).
 #include "pf_diffuse_common.h"
 
