@@ -920,7 +920,8 @@ int pf_create(const pf_desc *desc, pf_handle **out) {
     return rc;
   if ((rc = chk(hipMalloc(&h->flag, N), "alloc bulk flags")) != PF_OK) return rc;
   if ((rc = chk(hipMalloc(&h->unit, N), "alloc bulk flags")) != PF_OK) return rc;
-  if (use_direct(h.get(), h->NF) &&
+  // (six faces: the accelerator calls sum them on domains of one row as well, whose step has four)
+  if (use_direct(h.get(), 6) &&
       (rc = chk(hipMalloc(&h->packed, (N + 15) / 16 * 4), "alloc packed flags")) != PF_OK)
     return rc;
   if ((rc = chk(hipMalloc(&h->bulk_count, 4 * sizeof(unsigned)), "alloc bulk counts")) != PF_OK)
