@@ -29,10 +29,11 @@ __global__ __launch_bounds__(kTileNT) void diffuse_tile_kernel(
   constexpr int NF = 4, NT = kTileNT, V = kTileV, G = kTileG;
   constexpr int CELLS = NT * V, SLOTS = NT * G;
   constexpr int EXTRA = SLOTS * P > CELLS ? SLOTS * P : CELLS;
-  static_assert(CELLS + EXTRA < 65535, "16-bit element indices");
+  constexpr int NONE = CELLS + EXTRA;  // the partition of an absent phase
+  static_assert(NONE < 65535, "16-bit element indices");
   static_assert(V <= 8 && G * P <= 32, "packed codes and presence bits");
-  __shared__ A L[CELLS + EXTRA];       // the cells' values; behind them the entries' partitions (or,
-                                       // in a dense tile, the listed cells' new values)
+  __shared__ A L[NONE + 1];            // the cells' values; behind them the entries' partitions (or,
+                                       // in a dense tile, the listed cells' new values); 0
   __shared__ uint16_t slot_of[CELLS];  // a listed cell's entry, 0xffff for the others
   __shared__ uint16_t list[CELLS];     // the listed cells
   __shared__ uint8_t codes[F::kMixed ? CELLS : 1];
@@ -51,7 +52,10 @@ __global__ __launch_bounds__(kTileNT) void diffuse_tile_kernel(
   const int X = ibx + 2 * S, Y = iby + 2 * S, ncells = X * Y;
   const int ox = ix0 - S, oy = iy0 - S;
 
-  if (t == 0) counter = 0;
+  if (t == 0) {
+    counter = 0;
+    L[NONE] = A(0);
+  }
   __syncthreads();
 
   auto wrapn = [](int i, int e) {  // into [0, e), from any distance (a halo may span the domain)
@@ -173,7 +177,11 @@ __global__ __launch_bounds__(kTileNT) void diffuse_tile_kernel(
   if (ng <= SLOTS) {
     A w[G][NF * P], t1[G][P], t2[G][P], cp[G][P], sc[G];
     int sdepth[G];
-    uint32_t saddr[G][NF / 2], sgi[G], present = 0;  // saddr: places in L, two faces per word
+    // saddr: a neighbour's partition in L by face and phase, two places per word.  A bulk neighbour's
+    // is its value for the phase it has and 0 for the others (0 * (value - c) would be NaN once the
+    // value overflows).
+    static_assert(P * NF % 2 == 0, "two places per word");
+    uint32_t saddr[G][NF * P / 2], sgi[G], present = 0;
     CompCode sq[G];
     // partition_cell of an entry's value (the division by t1 = 1 of a unit cell changes nothing)
     auto partition = [&](int j) {
@@ -190,7 +198,8 @@ __global__ __launch_bounds__(kTileNT) void diffuse_tile_kernel(
       sq[j] = 0;
       sgi[j] = 0;
       sc[j] = A(0);
-      saddr[j][0] = saddr[j][1] = 0;
+#pragma unroll
+      for (int q = 0; q < NF * P / 2; ++q) saddr[j][q] = 0;
 #pragma unroll
       for (int p = 0; p < P; ++p) {
         t1[j][p] = A(1);
@@ -216,8 +225,14 @@ __global__ __launch_bounds__(kTileNT) void diffuse_tile_kernel(
         for (int f = 0; f < NF; ++f) {
           const int nidx = o.depth > 0 ? idx + o.off[f] : idx;
           const uint32_t s2 = slot_of[nidx];
-          const uint32_t a = s2 == 0xffffu ? uint32_t(nidx) : uint32_t(CELLS) + s2 * uint32_t(P);
-          saddr[j][f >> 1] |= a << (16 * (f & 1));
+#pragma unroll
+          for (int p = 0; p < P; ++p) {
+            const uint32_t a = s2 != 0xffffu      ? uint32_t(CELLS) + s2 * uint32_t(P) + uint32_t(p)
+                               : phn[f][p] > A(0) ? uint32_t(nidx)
+                                                  : uint32_t(NONE);
+            const int q = f * P + p;
+            saddr[j][q >> 1] |= a << (16 * (q & 1));
+          }
         }
 #pragma unroll
         for (int i = 0; i < P; ++i) {
@@ -252,18 +267,15 @@ __global__ __launch_bounds__(kTileNT) void diffuse_tile_kernel(
         if (waves_first + j * NT >= ng) break;  // wave-uniform
         DelAcc<F, P> acc;
 #pragma unroll
-        for (int f = 0; f < NF; ++f) {
-          const uint32_t a = (saddr[j][f >> 1] >> (16 * (f & 1))) & 0xffffu;
-          // a bulk neighbour's partition is its value for the one phase it has; the weights of the
-          // other phases are 0
-          const uint32_t step = a >= uint32_t(CELLS) ? 1u : 0u;
+        for (int f = 0; f < NF; ++f)
 #pragma unroll
           for (int p = 0; p < P; ++p) {
-            const A term = w[j][f * P + p] * (L[a + step * uint32_t(p)] - cp[j][p]);
+            const int q = f * P + p;
+            const uint32_t a = (saddr[j][q >> 1] >> (16 * (q & 1))) & 0xffffu;
+            const A term = w[j][q] * (L[a] - cp[j][p]);
             if (f == 0) acc.first(p, term, dc);
             else acc.add(p, term, dc);
           }
-        }
         const A del = acc.result(dc);
         A v;
         CompCode qo = 0;

@@ -1,0 +1,64 @@
+"""GPU: diffusion sub-steps of planes in which a concentration, or a phase's share of it, has overflowed:
+infinities and NaN stand where the full-formula kernel has them.  There an absent phase's partition is
+0; the oracle divides for absent phases too, so its 0 * (inf - c) is NaN where the kernels have 0."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch  # noqa: F401  (before the library: both then use one HIP runtime)
+
+import oracle
+from phasefield_amd import Domain
+from phasefield_amd._capi import PfParams
+from tests import helpers
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def params(tmp_path_factory):
+    m = helpers.small_model(str(tmp_path_factory.mktemp("nf")), "fec_3d_256", nx=16, ny=16, nz=16,
+                            grains=4, nuclei=2)
+    q = oracle.as_orc_params(helpers.model_params(m))
+    q.diffusivity[0][2] = 5.0
+    return q
+
+
+def ferrite(nx, ny, mixed_cells):
+    """Ferrite with half austenite in `mixed_cells`: these and their neighbours take the full formula."""
+    n = nx * ny
+    ids, val, phase = np.zeros((n, 4), np.int32), np.zeros((n, 4)), np.zeros((n, 3))
+    ids[:, 0], val[:, 0], phase[:, 1] = 200001, 1.0, 1.0
+    for c in mixed_cells:
+        ids[c, :2], val[c, :2], phase[c, :2] = (100001, 200001), 0.5, 0.5
+    conc = 0.02 + 0.8 * np.random.default_rng(21).random(n)
+    return ids.reshape(-1), val.reshape(-1), phase.reshape(-1), conc
+
+
+def different(a, b):
+    return np.flatnonzero(~((a == b) | (np.isnan(a) & np.isnan(b)))).tolist()
+
+
+@pytest.mark.parametrize("form", [oracle.ORC_FP64, oracle.ORC_MIXED])
+@pytest.mark.parametrize("P", [2, 3])
+@pytest.mark.parametrize("count", [1, 3])
+def test_overflowed_bulk_neighbour(P, form, count, params, monkeypatch):
+    """A listed cell next to a bulk cell of infinite concentration."""
+    print(f"[gpu] overflowed bulk neighbour P={P} form={form} count={count}", flush=True)
+    nx, ny = 40, 24
+    state = ferrite(nx, ny, [10 + nx * 10])
+    state[3][8 + nx * 10] = np.inf  # bulk; its neighbour at x = 9 is listed
+    q = PfParams.from_buffer_copy(params)
+    q.dims = 2
+    conc = []
+    for kernel in ("lds", "bulk"):
+        monkeypatch.setenv("PFAMD_DIFF_KERNEL", kernel)
+        g = Domain(nx, ny, 1, depth=4, nphase=P,
+                   precision="mixed" if form == oracle.ORC_MIXED else "fp64")
+        g.set_params(q)
+        g.upload(*state)
+        g.diffuse(0, count, q.dt_d[0])
+        conc.append(g.download()["conc"])
+        g.close()
+    assert np.isinf(conc[0]).any() and np.isnan(conc[0]).any() and np.isfinite(conc[0]).any()
+    assert different(conc[1], conc[0]) == []
