@@ -705,15 +705,15 @@ bool tile_geom(const pf_handle *h, int left, TileGeom &g) {
   return tile_geometry(h->d.nx, h->d.ny, h->d.nz, left, h->tile_pin, g);
 }
 
-template <class F, int P, int NF, bool NOF>
+template <class F, int P, int NF>
 hipError_t launch_tile(pf_handle *h, int s, const DiffConsts<typename F::A> &dc,
                        const TileGeom &g) {
   using T = typename F::T;
   using C = typename F::C;
-  const hipError_t e = ensure_flags<T, P, NF, NOF>(h);
+  const hipError_t e = ensure_flags<T, P, NF, false>(h);
   if (e != hipSuccess) return e;
   const int a = h->ccur[s], b = 1 - a;
-  hipLaunchKernelGGL((diffuse_tile_kernel<F, P>), dim3(unsigned(g.nblocks)), dim3(kTileNT), 0,
+  hipLaunchKernelGGL((diffuse_tile_kernel<F, P, NF == 6>), dim3(unsigned(g.nblocks)), dim3(kTileNT), 0,
                      h->stream, static_cast<const C *>(h->conc[s][a]),
                      static_cast<C *>(h->conc[s][b]), static_cast<const T *>(h->pfrac), h->flag, dc,
                      g, h->N, h->csub[s], s);
@@ -724,8 +724,10 @@ hipError_t launch_tile(pf_handle *h, int s, const DiffConsts<typename F::A> &dc,
 template <class F, int P>
 hipError_t dispatch_tile_p(pf_handle *h, int s, const DiffConsts<typename F::A> &dc,
                            const TileGeom &g) {
-  if (h->NF == 4) return launch_tile<F, P, 4, false>(h, s, dc, g);
-  return launch_tile<F, P, 6, false>(h, s, dc, g);  // one plane: its z faces carry no flux
+  // six faces on one plane: the accelerator call, FP64 with three phases
+  if constexpr (P == 3 && !F::kMixed)
+    if (h->NF == 6) return launch_tile<F, P, 6>(h, s, dc, g);
+  return launch_tile<F, P, 4>(h, s, dc, g);
 }
 
 template <class F, int P>

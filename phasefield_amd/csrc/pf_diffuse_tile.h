@@ -49,7 +49,8 @@ inline bool tile_geometry(int nx, int ny, int nz, int left, const int *pin, Tile
   return nblocks <= 0x7fffffffL && (g.bx + 2 * steps) * (g.by + 2 * steps) <= kTileNT * kTileV;
 }
 
-template <class F, int P>
+// SELF_Z: z faces that join each cell to itself (six-face calls on one plane).
+template <class F, int P, bool SELF_Z>
 __global__ void diffuse_tile_kernel(const typename F::C *__restrict__ cin,
                                     typename F::C *__restrict__ cout,
                                     const typename F::T *__restrict__ pfrac,

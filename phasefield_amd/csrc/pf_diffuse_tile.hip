@@ -14,12 +14,13 @@
 // them from memory instead (the full formula, every sub-step).
 //
 // A one-cell-thick domain whose stencil has six faces (the accelerator calls) runs here as well: its
-// z faces join a cell to itself and carry no flux.
+// z faces join a cell to itself and carry no flux, only the NaN of a partition that is not finite
+// (SELF_Z; an infinite bulk cell becomes NaN without them).
 #include "pf_diffuse_tile.h"
 
 namespace pfamd {
 
-template <class F, int P>
+template <class F, int P, bool SELF_Z>
 __global__ __launch_bounds__(kTileNT) void diffuse_tile_kernel(
     const typename F::C *__restrict__ cin, typename F::C *__restrict__ cout,
     const typename F::T *__restrict__ pfrac, const uint8_t *__restrict__ flag,
@@ -152,6 +153,14 @@ __global__ __launch_bounds__(kTileNT) void diffuse_tile_kernel(
     for (int k = 0; k < V; ++k)
       if (depth[k] >= s) L[t + k * NT] = nv[k];
   };
+  // what faces that join a cell to itself add: 0, or NaN where a partition is not finite
+  static_assert(!SELF_Z || !F::kMixed, "an FP64 sum starts from it");
+  auto self_z = [](const auto &c) {
+    A z = c[0] * A(0);
+#pragma unroll
+    for (int p = 1; p < P; ++p) z = __builtin_elementwise_fma(c[p], A(0), z);
+    return z;
+  };
   // a listed cell's place, its neighbours' in the domain and in L, and its depth
   struct Cell {
     uint32_t g, gn[4];
@@ -266,6 +275,7 @@ __global__ __launch_bounds__(kTileNT) void diffuse_tile_kernel(
       for (int j = 0; j < G; ++j) {
         if (waves_first + j * NT >= ng) break;  // wave-uniform
         DelAcc<F, P> acc;
+        if constexpr (SELF_Z) acc.s[0] = self_z(cp[j]);
 #pragma unroll
         for (int f = 0; f < NF; ++f)
 #pragma unroll
@@ -320,13 +330,21 @@ __global__ __launch_bounds__(kTileNT) void diffuse_tile_kernel(
           st.me.c = typename F::C(v);
 #pragma unroll
           for (int p = 0; p < P; ++p) st.me.ph[p] = pfrac[long(o.g) * P + p];
+          A z = A(0);
+          if constexpr (SELF_Z) {  // (before the neighbours are loaded: registers)
+            CellPF<A> me;
+            partition_cell<F, P>(st.me, dc, me);
+            z = self_z(me.c);
+            asm volatile("" : "+v"(z));
+          }
 #pragma unroll
           for (int f = 0; f < NF; ++f) {
             st.nb[f].c = typename F::C(L[idx + o.off[f]]);
 #pragma unroll
             for (int p = 0; p < P; ++p) st.nb[f].ph[p] = pfrac[long(o.gn[f]) * P + p];
           }
-          const A del = stencil_del<F, P, NF>(st, dc);
+          A del = stencil_del<F, P, NF>(st, dc);
+          if constexpr (SELF_Z) del += z;
           if constexpr (F::kMixed) {
             CompCode qo;
             v = mixed_step(v, del, comp_unpack(codes[idx]), comp_hash(o.g, key), qo);
@@ -372,13 +390,14 @@ __global__ __launch_bounds__(kTileNT) void diffuse_tile_kernel(
   }
 }
 
-#define PF_INST_TILE(F, P)                                                                       \
-  template __global__ void diffuse_tile_kernel<F, P>(const F::C *, F::C *, const F::T *,         \
-                                                     const uint8_t *, const DiffConsts<F::A>,    \
-                                                     TileGeom, long, uint32_t, int);
-PF_INST_TILE(FormF64, 2)
-PF_INST_TILE(FormF64, 3)
-PF_INST_TILE(FormMixed, 2)
-PF_INST_TILE(FormMixed, 3)
+#define PF_INST_TILE(F, P, SELF_Z)                                                              \
+  template __global__ void diffuse_tile_kernel<F, P, SELF_Z>(                                   \
+      const F::C *, F::C *, const F::T *, const uint8_t *, const DiffConsts<F::A>, TileGeom,     \
+      long, uint32_t, int);
+PF_INST_TILE(FormF64, 2, false)
+PF_INST_TILE(FormF64, 3, false)
+PF_INST_TILE(FormF64, 3, true)
+PF_INST_TILE(FormMixed, 2, false)
+PF_INST_TILE(FormMixed, 3, false)
 
 }  // namespace pfamd

@@ -150,8 +150,7 @@ extern "C" int pf_gpu_diffusion_solver_noalloc(const double *hdiffusivity,
   if (z == 1 && tile_geometry(x, y, 1, num_loop, nullptr, tile)) {
     for (int left = num_loop; left > 0; left -= tile.steps) {
       (void)tile_geometry(x, y, 1, left, nullptr, tile);
-      // (the z faces of a one-cell-thick domain carry no flux)
-      hipLaunchKernelGGL((diffuse_tile_kernel<FormF64, 3>), dim3(unsigned(tile.nblocks)),
+      hipLaunchKernelGGL((diffuse_tile_kernel<FormF64, 3, true>), dim3(unsigned(tile.nblocks)),
                          dim3(kTileNT), 0, s, a, b, pf, buf.flag, dc, tile, N, 0u, 0);
       std::swap(a, b);
     }

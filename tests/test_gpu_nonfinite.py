@@ -3,12 +3,14 @@ infinities and NaN stand where the full-formula kernel has them.  There an absen
 0; the oracle divides for absent phases too, so its 0 * (inf - c) is NaN where the kernels have 0."""
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
-import torch  # noqa: F401  (before the library: both then use one HIP runtime)
+import torch  # before the library: both then use one HIP runtime
 
 import oracle
-from phasefield_amd import Domain
+from phasefield_amd import Domain, gpu_cleanup, gpu_diffusion_solver, lib
 from phasefield_amd._capi import PfParams
 from tests import helpers
 
@@ -62,3 +64,39 @@ def test_overflowed_bulk_neighbour(P, form, count, params, monkeypatch):
         g.close()
     assert np.isinf(conc[0]).any() and np.isnan(conc[0]).any() and np.isfinite(conc[0]).any()
     assert different(conc[1], conc[0]) == []
+
+
+@pytest.mark.parametrize("loops", [1, 3])
+def test_overflowed_partition_of_a_plane_with_six_faces(loops, params):
+    """The accelerator calls sum six faces also where z is one cell: a phase whose partitioned
+    concentration overflows gives inf - inf on the faces that join the cell to itself."""
+    print(f"[gpu] overflowed partition, six faces, loops={loops}", flush=True)
+    stream = torch.cuda.current_stream().cuda_stream
+    nx, ny = 40, 24
+    cell = 10 + nx * 10
+    ids, val, phase, conc = ferrite(nx, ny, [cell, cell - 1, cell + 1, cell - nx, cell + nx])
+    conc[cell] = 1.5e308
+    q = PfParams.from_buffer_copy(params)
+    q.dims = 3
+    q.part_k[0][0][1] = 0.1  # austenite's partition of the cell: c / 0.55
+    D = np.array([q.diffusivity[0][i] for i in range(3)])
+    pk = np.array([[q.part_k[0][i][j] for j in range(3)] for i in range(3)]).T.reshape(-1).copy()
+    pc = np.array([[q.part_c[0][i][j] for j in range(3)] for i in range(3)]).T.reshape(-1).copy()
+    dt = (loops - 0.1) * (q.dx * q.dx / D.max() / 2 * float(np.float32(0.2)))
+    o = oracle.OracleDomain(nx, ny, 1, 4, 1)
+    o.set_params(oracle.as_orc_params(q))
+    o.set_state(ids, val, phase, conc)
+    o.diffuse_factor(0, loops, dt / loops / (q.dx * q.dx))
+    want = o.get_state()["conc"]
+    assert np.isnan(want[cell]) and np.isfinite(want).any()
+    host = conc.copy()
+    gpu_diffusion_solver(D, pk, pc, phase, host, nx, ny, 1, dt, q.dx)
+    gpu_cleanup()
+    dphase = torch.from_numpy(phase).to("cuda:0")
+    dconc = torch.from_numpy(conc).to("cuda:0")
+    ptr = [a.ctypes.data_as(ctypes.POINTER(ctypes.c_double)) for a in (D, pk, pc)]
+    rc = lib().pf_gpu_diffusion_solver_noalloc(*ptr, dphase.data_ptr(), dconc.data_ptr(), nx, ny, 1, dt,
+                                               q.dx, stream)
+    assert rc == 0, lib().pf_last_error(None)
+    assert different(dconc.cpu().numpy(), want) == []
+    assert different(host, want) == []
