@@ -702,7 +702,7 @@ hipError_t launch_diffuse(pf_handle *h, int s, const DiffConsts<typename F::A> &
 // single-sub-step kernels run.
 bool tile_geom(const pf_handle *h, int left, TileGeom &g) {
   if (!h->diff_tile || !(h->NF == 4 || h->d.nz == 1) || !default_diffusion(h)) return false;
-  return tile_geometry(h->d.nx, h->d.ny, h->d.nz, left, h->tile_pin, g);
+  return tile_geometry(h->d.nx, h->d.ny, h->d.nz, is_mixed(h), left, h->tile_pin, g);
 }
 
 template <class F, int P, int NF>

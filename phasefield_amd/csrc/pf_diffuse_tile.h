@@ -1,5 +1,7 @@
 // pf_diffuse_tile.h — several diffusion sub-steps per launch on planes (pf_diffuse_tile.hip).
 #pragma once
+#include <algorithm>
+
 #include "pf_diffuse_common.h"
 
 namespace pfamd {
@@ -24,9 +26,23 @@ struct TileGeom {
 //   256^2:     16 x 16, 12: 1.42; 16 x 16, 8: 1.52; 32 x 16, 10: 1.6
 //   512^2:     32 x 32, 6: 2.30; 24 x 24, 10: 2.97; 20 x 20, 12: 3.75
 //   1000 x 600: 32 x 32, 6: 4.89 (single sub-steps: 10.9)
-// so tiles grow once they outnumber the compute units.  Above about 1.5 M cells the planes fill the
-// chip by themselves and single sub-steps, which compute no halo, win.
-inline bool tile_geometry(int nx, int ny, int nz, int left, const int *pin, TileGeom &g) {
+// so tiles grow once they outnumber the compute units.
+//
+// Tiles are taken as long as what they compute, halo included, is at most 2.2 M cells (mixed 3.5 M) or
+// 2.1 times the domain.  A step with single sub-steps / with tiles, three domains in turn (one domain
+// alone gains more):
+//                                  FP64            mixed
+//   1024^2 (2.0 M computed)        1.55 / 1.20     1.40 / 0.83 ms
+//   1224^2 (2.9 M)                 1.85 / 1.68     1.50 / 1.17
+//   160 x 1 x 160 (1.6 M)          1.19 / 0.80     1.18 / 0.54
+//   200 x 1 x 200 (2.6 M)          1.14 / 1.27     1.17 / 0.86
+//   230 x 1 x 230 (3.5 M)          1.15 / 1.66     1.13 / 1.13
+//   300 x 1 x 300 (5.7 M)          1.44 / 2.74     1.44 / 1.86
+//   1000 x 1 x 600 (10.7 M)        1.66 / 10.5     1.57 / 7.40
+// (a row one cell wide is its own halo in y, `steps` times over on either side).  Planes above 1.5 M
+// cells keep single sub-steps; tiles of 32 x 32 and 6 sub-steps would gain there as well up to about
+// 6 M cells (1500^2 FP64 2.57 / 2.42) and lose at 4096^2 (16.3 / 18.3).
+inline bool tile_geometry(int nx, int ny, int nz, bool mixed, int left, const int *pin, TileGeom &g) {
   const long n = long(nx) * ny * nz;
   int bx = 32, by = 32, steps = 6;
   if (n <= 8192) bx = by = steps = 8;
@@ -43,6 +59,9 @@ inline bool tile_geometry(int nx, int ny, int nz, int left, const int *pin, Tile
   split(nx, bx, g.bx, g.nbx);
   split(ny, by, g.by, g.nby);
   const long nblocks = long(g.nbx) * g.nby * nz;
+  if (!(pin && pin[2] > 0) &&
+      double(nblocks) * (g.bx + 2 * steps) * (g.by + 2 * steps) > std::max(mixed ? 3.5e6 : 2.2e6, 2.1 * double(n)))
+    return false;
   const int launches = (left + steps - 1) / steps;
   g.nblocks = int(nblocks);
   g.steps = (left + launches - 1) / launches;

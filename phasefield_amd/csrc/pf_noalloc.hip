@@ -147,9 +147,9 @@ extern "C" int pf_gpu_diffusion_solver_noalloc(const double *hdiffusivity,
     return set_global_error(PF_ERR_HIP, std::string("pf_gpu_diffusion_solver_noalloc: launch: ") +
                                             hipGetErrorString(e));
   TileGeom tile;
-  if (z == 1 && tile_geometry(x, y, 1, num_loop, nullptr, tile)) {
+  if (z == 1 && tile_geometry(x, y, 1, false, num_loop, nullptr, tile)) {
     for (int left = num_loop; left > 0; left -= tile.steps) {
-      (void)tile_geometry(x, y, 1, left, nullptr, tile);
+      (void)tile_geometry(x, y, 1, false, left, nullptr, tile);
       hipLaunchKernelGGL((diffuse_tile_kernel<FormF64, 3, true>), dim3(unsigned(tile.nblocks)),
                          dim3(kTileNT), 0, s, a, b, pf, buf.flag, dc, tile, N, 0u, 0);
       std::swap(a, b);
