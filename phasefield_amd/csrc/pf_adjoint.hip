@@ -842,15 +842,15 @@ template <int K, int P, int NF, bool NOF> struct Adj {
           if (vec && mby == 8)
             hipLaunchKernelGGL((diffuse_bulk_march_kernel<FormF64, P, NF, NOF, 8, 2, 1>),
                                dim3(mnb), dim3(64, 8), 0, st, lam_c, lam_c2, sd.count, dc, v.nx,
-                               v.ny, v.nz, mzc, mtx, mty, int(mnb), (s & 1) != 0);
+                               v.ny, v.nz, mzc, mtx, mty, int(mnb));
           else if (vec && mby == 16)
             hipLaunchKernelGGL((diffuse_bulk_march_kernel<FormF64, P, NF, NOF, 16, 2, 1>),
                                dim3(mnb), dim3(64, 16), 0, st, lam_c, lam_c2, sd.count, dc, v.nx,
-                               v.ny, v.nz, mzc, mtx, mty, int(mnb), (s & 1) != 0);
+                               v.ny, v.nz, mzc, mtx, mty, int(mnb));
           else if (vec && mby == 32)
             hipLaunchKernelGGL((diffuse_bulk_march_kernel<FormF64, P, NF, NOF, 32, 2, 2>),
                                dim3(mnb), dim3(64, 16), 0, st, lam_c, lam_c2, sd.count, dc, v.nx,
-                               v.ny, v.nz, mzc, mtx, mty, int(mnb), (s & 1) != 0);
+                               v.ny, v.nz, mzc, mtx, mty, int(mnb));
           else if (vec)
             hipLaunchKernelGGL((diffuse_bulk_vec_kernel<FormF64, P, NF, NOF, 4, 2>),
                                dim3(gvec.nblocks), dim3(64, 4), 0, st, lam_c, lam_c2, sd.flag, dc,

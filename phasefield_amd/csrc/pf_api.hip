@@ -85,7 +85,7 @@ struct pf_handle {
   bool diff_march = true;    // ... in its plane-marching form
   int march_by = 0;          // its tile rows and z-chunk, picked by timing at first use
   int march_zc = 0;
-  bool flip = false;         // direction of the next bulk pass (alternates)
+  bool flip = false;         // direction of the direct kernel's next pass (alternates)
   int *list_len = nullptr;   // [0]: cells the last sweep listed, [1]: cells the diffusion lists
   int *ccount = nullptr;     // pair lists: listed cells per list block ([nblocks + 1])
   bool ccount_pending = false;  // ccount not yet summed into list_len[1]
@@ -443,7 +443,7 @@ hipError_t launch_march(pf_handle *h, const DiffConsts<typename F::A> &dc,
       constexpr int BY = decltype(rows)::value, R = decltype(per_wave)::value;
       hipLaunchKernelGGL((diffuse_bulk_march_kernel<F, P, NF, NOF, BY, V, R>), dim3(nblocks),
                          dim3(64, BY / R), 0, h->stream, cin, cout, h->bulk_count, dc, nx, ny, nz,
-                         zc, tiles_x, tiles_y, int(nblocks), h->flip);
+                         zc, tiles_x, tiles_y, int(nblocks));
     };
     using std::integral_constant;
     if (by == 8) go(integral_constant<int, 8>(), integral_constant<int, 1>());
@@ -520,9 +520,7 @@ hipError_t launch_march(pf_handle *h, const DiffConsts<typename F::A> &dc,
       }
     }
   }
-  const hipError_t e = launch(h->march_by, h->march_zc);
-  h->flip = !h->flip;  // the next sub-step starts where this one ended
-  return e;
+  return launch(h->march_by, h->march_zc);
 }
 
 // whether the single sub-steps run the plane-marching kernel (which addresses a plane with 32-bit

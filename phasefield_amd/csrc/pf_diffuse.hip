@@ -702,7 +702,7 @@ __global__ __launch_bounds__(64 * BY / R) void diffuse_bulk_march_kernel(
     const typename F::C *__restrict__ cin, typename F::C *__restrict__ cout,
     const unsigned *__restrict__ count, const DiffConsts<typename F::A> dc, const int nx,
     const int ny, const int nz, const int zchunk, const int tiles_x, const int tiles_y,
-    const int nblocks, const bool flip) {
+    const int nblocks) {
   using A = typename F::A;
   using VA = VecA<A, V>;
   static_assert(BY % R == 0, "rows per wavefront must divide the tile height");
@@ -722,8 +722,7 @@ __global__ __launch_bounds__(64 * BY / R) void diffuse_bulk_march_kernel(
   __shared__ VA s[2][BY][64];
   const int b = blockIdx.x;
   const int per = nblocks >> 3, rem = nblocks & 7, xcd = b & 7;
-  const int mine = per + (xcd < rem ? 1 : 0);
-  const int logical = xcd * per + (xcd < rem ? xcd : rem) + (flip ? mine - 1 - (b >> 3) : b >> 3);
+  const int logical = xcd * per + (xcd < rem ? xcd : rem) + (b >> 3);
   const int tx_t = logical % tiles_x;
   const int t2 = logical / tiles_x;
   const int ty_t = t2 % tiles_y;
@@ -1425,7 +1424,7 @@ PF_INST_CLASSIFY(float, 3)
 #define PF_INST_MARCH_ONE(F, P, NF, NOF, BY, V, R)                                                 \
   template __global__ void diffuse_bulk_march_kernel<F, P, NF, NOF, BY, V, R>(                     \
       const F::C *, F::C *, const unsigned *, const DiffConsts<F::A>, int, int, int, int, int,    \
-      int, int, bool);
+      int, int);
 #define PF_INST_MARCH_NF(F, P, BY, V, R)          \
   PF_INST_MARCH_ONE(F, P, 4, false, BY, V, R)     \
   PF_INST_MARCH_ONE(F, P, 6, false, BY, V, R)     \

@@ -89,8 +89,7 @@ __global__ void diffuse_bulk_march_kernel(const typename F::C *__restrict__ cin,
                                           const unsigned *__restrict__ count,
                                           const DiffConsts<typename F::A> dc, const int nx,
                                           const int ny, const int nz, const int zchunk,
-                                          const int tiles_x, const int tiles_y, const int nblocks,
-                                          const bool flip);
+                                          const int tiles_x, const int tiles_y, const int nblocks);
 
 template <class F, int P, int NF, bool NOFLUX>
 __global__ void diffuse_general_kernel(const typename F::C *__restrict__ cin,
