@@ -203,8 +203,13 @@ typedef struct pf_adjoint_result {
 } pf_adjoint_result;
 
 /* Run forward with checkpoints from the current state, then the reverse sweep.  The device
- * state after the call is the final forward state. */
+ * state after the call is the final forward state.  A run's device memory of up to 16 GiB (128^3,
+ * 3 steps: 8.5 GB) stays with the handle for its next run; it is given back by pf_adjoint_release,
+ * with the handle, and when another call of this library finds the device full. */
 int pf_adjoint_run(pf_handle *h, const pf_adjoint_spec *spec, pf_adjoint_result *out);
+/* Give back the device memory that the handle's adjoint runs keep (for other allocators of the
+ * process); the next run allocates it again. */
+int pf_adjoint_release(pf_handle *h);
 
 /* ---- host model: input files, temperature path, parameter update ---------------------------- */
 

@@ -262,7 +262,8 @@ class Domain:
                + weight_conc * ||c_final - target_conc||^2.
         Returns the loss, the forward f_gamma samples and dL/d(mobility scale),
         dL/d(interface-energy scale), dL/dD(phase 1, carbon) and dL/dc0 (carbon, per cell).
-        The domain holds the final forward state afterwards.
+        The domain holds the final forward state afterwards, and up to 16 GiB of device memory for
+        its next run (adjoint_release gives it back).
         """
         samples = list(sample_steps)
         targets = list(target_fraction)
@@ -290,6 +291,10 @@ class Domain:
                 "d_mobility": res.d_mobility, "d_sigma": res.d_sigma,
                 "d_diff_gamma": res.d_diff_gamma, "d_conc0": g,
                 "forward_ms": res.forward_ms, "reverse_ms": res.reverse_ms}
+
+    def adjoint_release(self) -> None:
+        """Give back the device memory kept between adjoint runs."""
+        _check(lib().pf_adjoint_release(self._h), self._h, "pf_adjoint_release")
 
 
 class Model:

@@ -100,6 +100,7 @@ SIGNATURES = {
     "pf_copy_state": (_I, [_H, _H]),
     "pf_rex_fraction": (_I, [_H, C.POINTER(_D)]),
     "pf_adjoint_run": (_I, [_H, C.POINTER(PfAdjointSpec), C.POINTER(PfAdjointResult)]),
+    "pf_adjoint_release": (_I, [_H]),
     "pf_model_read": (_I, [C.c_char_p, C.POINTER(_M)]),
     "pf_model_free": (_I, [_M]),
     "pf_model_last_error": (C.c_char_p, []),

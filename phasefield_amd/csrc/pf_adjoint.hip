@@ -563,7 +563,8 @@ struct Arena {
     return d;
   }
 };
-// A block of at most this many bytes stays with the handle between runs.  Allocating and freeing it each
+// A block of at most this many bytes stays with the handle between runs, until the handle ends, the
+// caller gives it back (pf_adjoint_release) or another allocation needs it.  Allocating and freeing it each
 // run took 10 of 43 ms (128^3, 3 steps: 8.5 GB), and freed memory is cleared before it is handed out
 // again, which stalled runs in quick succession to 220 ms and some to seconds.
 constexpr size_t kKeptBlock = size_t(16) << 30;
@@ -677,7 +678,7 @@ template <int K, int P, int NF, bool NOF> struct Adj {
     const hipError_t mem_err = hipMemGetInfo(&mem_free, &mem_total);
     if (mem_err != hipSuccess)
       return handle_fail(h, PF_ERR_HIP, std::string("adjoint: ") + hipGetErrorString(mem_err));
-    const double left = double(mem_free) + double(handle_adjoint_kept(h)) - double(fixed.used);
+    const double left = double(mem_free) + double(handle_adjoint_idle(h)) - double(fixed.used);
     const char *env = std::getenv("PFAMD_ADJ_RECOMPUTE");
     const bool force_step = env && std::strcmp(env, "step") == 0;
     const bool store_segment = !force_step && double(per_step) * CK < 0.8 * left;
@@ -688,17 +689,15 @@ template <int K, int P, int NF, bool NOF> struct Adj {
     layout(ar, nstore, nckpt);
     const size_t bytes = ar.used;
     ar = Arena{};
-    ar.base = static_cast<char *>(handle_adjoint_block(h, bytes));
+    ar.base = static_cast<char *>(handle_adjoint_take(h, bytes));
     if (!ar.base) {
       (void)hipGetLastError();
       return handle_fail(h, PF_ERR_OOM, "adjoint buffers: out of memory");
     }
     layout(ar, nstore, nckpt);
-    struct Release {  // large blocks go back after the run
+    struct Release {  // the block goes back after the run, or stays with the handle
       pf_handle *h;
-      ~Release() {
-        if (handle_adjoint_kept(h) > kKeptBlock) handle_adjoint_release(h);
-      }
+      ~Release() { handle_adjoint_done(h, kKeptBlock); }
     } release{h};
 
     // first error of the asynchronous copies and clears below (reported by launch_ok)

@@ -21,6 +21,7 @@
 #include "pf_diffuse_direct.h"
 #include "pf_diffuse_tile.h"
 #include "pf_handle_access.h"
+#include "pf_kept_blocks.h"
 #include "pf_kernels.h"
 
 using namespace pfamd;
@@ -111,8 +112,6 @@ struct pf_handle {
   // next sub-step of solute s mixes two tables: 1 = the cells the last sweep copied keep the
   // previous ones, 2 = every cell does (no sweep since the change)
   int retable[PF_MAX_SOLUTE] = {0, 0};
-  void *adj_block = nullptr;  // the adjoint's device memory (handle_adjoint_block)
-  size_t adj_bytes = 0;
   // asynchronous VTI dump: device fields -> pinned host copy (dump stream) -> writer thread
   void *dump_dev = nullptr;      // korn [N] int32, conc [N] float
   void *dump_host = nullptr;     // pinned copy of dump_dev
@@ -141,6 +140,28 @@ int fail(pf_handle *h, int code, const std::string &msg) {
       return fail((h), e_ == hipErrorOutOfMemory ? PF_ERR_OOM : PF_ERR_HIP,                  \
                   std::string(#call) + ": " + hipGetErrorString(e_));                        \
   } while (0)
+
+// device memory that the handles' adjoint runs keep (never destroyed: handles may end after it would be)
+struct DeviceMem {
+  static void *alloc(size_t bytes) {
+    void *p = nullptr;
+    return hipMalloc(&p, bytes) == hipSuccess ? p : nullptr;
+  }
+  static void free(void *p) { (void)hipFree(p); }
+};
+KeptBlocks<DeviceMem> &kept_blocks() {
+  static KeptBlocks<DeviceMem> &blocks = *new KeptBlocks<DeviceMem>();
+  return blocks;
+}
+// hipMalloc that takes back what adjoint runs keep idle before it reports a full device
+template <class T> hipError_t device_malloc(T **p, size_t bytes) {
+  const hipError_t e = hipMalloc(p, bytes);
+  int dev = 0;
+  if (e != hipErrorOutOfMemory || hipGetDevice(&dev) != hipSuccess || !kept_blocks().release(dev))
+    return e;
+  (void)hipGetLastError();
+  return hipMalloc(p, bytes);
+}
 
 bool is_mixed(const pf_handle *h) { return h->d.precision == PF_MIXED; }
 
@@ -814,7 +835,7 @@ void free_all(pf_handle *h) {
   if (h->olist) hipFree(h->olist);
   if (h->gblock) hipFree(h->gblock);
   if (h->packed) hipFree(h->packed);
-  if (h->adj_block) hipFree(h->adj_block);
+  kept_blocks().drop(h, true);
   if (h->red) hipFree(h->red);
   for (int k = 0; k < 3; ++k)
     for (auto &pr : h->ev[k]) {
@@ -911,40 +932,40 @@ int pf_create(const pf_desc *desc, pf_handle **out) {
     return rc;
   const size_t N = size_t(h->N);
   for (int b = 0; b < 2; ++b) {
-    if ((rc = chk(hipMalloc(&h->id[b], N * h->KI * 2), "alloc ids")) != PF_OK) return rc;
-    if ((rc = chk(hipMalloc(&h->phi[b], N * d.depth * h->tsz), "alloc phi")) != PF_OK) return rc;
+    if ((rc = chk(device_malloc(&h->id[b], N * h->KI * 2), "alloc ids")) != PF_OK) return rc;
+    if ((rc = chk(device_malloc(&h->phi[b], N * d.depth * h->tsz), "alloc phi")) != PF_OK) return rc;
     for (int s = 0; s < d.nsolute; ++s)
-      if ((rc = chk(hipMalloc(&h->conc[s][b], h->cbuf), "alloc conc")) != PF_OK) return rc;
+      if ((rc = chk(device_malloc(&h->conc[s][b], h->cbuf), "alloc conc")) != PF_OK) return rc;
   }
-  if ((rc = chk(hipMalloc(&h->pfrac, N * d.nphase * h->tsz), "alloc value_phase")) != PF_OK)
+  if ((rc = chk(device_malloc(&h->pfrac, N * d.nphase * h->tsz), "alloc value_phase")) != PF_OK)
     return rc;
-  if ((rc = chk(hipMalloc(&h->flag, N), "alloc bulk flags")) != PF_OK) return rc;
-  if ((rc = chk(hipMalloc(&h->unit, N), "alloc bulk flags")) != PF_OK) return rc;
+  if ((rc = chk(device_malloc(&h->flag, N), "alloc bulk flags")) != PF_OK) return rc;
+  if ((rc = chk(device_malloc(&h->unit, N), "alloc bulk flags")) != PF_OK) return rc;
   // (six faces: the accelerator calls sum them on domains of one row as well, whose step has four)
   if (use_direct(h.get(), 6) &&
-      (rc = chk(hipMalloc(&h->packed, (N + 15) / 16 * 4), "alloc packed flags")) != PF_OK)
+      (rc = chk(device_malloc(&h->packed, (N + 15) / 16 * 4), "alloc packed flags")) != PF_OK)
     return rc;
-  if ((rc = chk(hipMalloc(&h->bulk_count, 4 * sizeof(unsigned)), "alloc bulk counts")) != PF_OK)
+  if ((rc = chk(device_malloc(&h->bulk_count, 4 * sizeof(unsigned)), "alloc bulk counts")) != PF_OK)
     return rc;
-  if ((rc = chk(hipMalloc(&h->glist, N * 4), "alloc full-formula list")) != PF_OK) return rc;
-  if ((rc = chk(hipMalloc(&h->list_len, 2 * sizeof(int)), "alloc list lengths")) != PF_OK) return rc;
-  if ((rc = chk(hipMalloc(&h->ccount, (list_blocks(h->N) + 1) * sizeof(int)), "alloc list counts")) !=
+  if ((rc = chk(device_malloc(&h->glist, N * 4), "alloc full-formula list")) != PF_OK) return rc;
+  if ((rc = chk(device_malloc(&h->list_len, 2 * sizeof(int)), "alloc list lengths")) != PF_OK) return rc;
+  if ((rc = chk(device_malloc(&h->ccount, (list_blocks(h->N) + 1) * sizeof(int)), "alloc list counts")) !=
       PF_OK)
     return rc;
   if ((rc = chk(hipMemsetAsync(h->list_len, 0, 2 * sizeof(int), h->stream), "clear")) != PF_OK)
     return rc;
-  if ((rc = chk(hipMalloc(&h->sflag, N), "alloc sweep copy flags")) != PF_OK) return rc;
-  if ((rc = chk(hipMalloc(&h->squeue, 8 * 32 * sizeof(int)), "alloc sweep counters")) != PF_OK)
+  if ((rc = chk(device_malloc(&h->sflag, N), "alloc sweep copy flags")) != PF_OK) return rc;
+  if ((rc = chk(device_malloc(&h->squeue, 8 * 32 * sizeof(int)), "alloc sweep counters")) != PF_OK)
     return rc;
   if (d.depth == 4 && !is_mixed(h.get()) &&
-      (rc = chk(hipMalloc(&h->olist, (h->N + 4) * sizeof(int)), "alloc sweep overflow list")) !=
+      (rc = chk(device_malloc(&h->olist, (h->N + 4) * sizeof(int)), "alloc sweep overflow list")) !=
           PF_OK)
     return rc;
-  if ((rc = chk(hipMalloc(&h->gblock, (list_blocks(h->N) + 1) * sizeof(int)),
+  if ((rc = chk(device_malloc(&h->gblock, (list_blocks(h->N) + 1) * sizeof(int)),
                 "alloc list offsets")) != PF_OK)
     return rc;
   h->red_blocks = int(std::min<long>(1024, std::max<long>(1, (h->N + 4095) / 4096)));
-  if ((rc = chk(hipMalloc(&h->red, sizeof(RedPartial) * h->red_blocks), "alloc partials")) != PF_OK)
+  if ((rc = chk(device_malloc(&h->red, sizeof(RedPartial) * h->red_blocks), "alloc partials")) != PF_OK)
     return rc;
   for (int b = 0; b < 2; ++b) {
     if ((rc = chk(hipMemsetAsync(h->id[b], 0, N * h->KI * 2, h->stream), "clear")) != PF_OK)
@@ -984,7 +1005,7 @@ int pf_dump_vti_async(pf_handle *h, const char *path, double dx) {
   hipSetDevice(h->d.device);
   const long N = h->N;
   if (!h->dump_dev) {
-    HIPCHK(h, hipMalloc(&h->dump_dev, size_t(N) * 8));
+    HIPCHK(h, device_malloc(&h->dump_dev, size_t(N) * 8));
     HIPCHK(h, hipHostMalloc(&h->dump_host, size_t(N) * 8, hipHostMallocDefault));
     HIPCHK(h, hipStreamCreateWithFlags(&h->dump_stream, hipStreamNonBlocking));
     HIPCHK(h, hipEventCreateWithFlags(&h->dump_ev[0], hipEventDisableTiming));
@@ -1358,6 +1379,13 @@ int pf_march_shape(const pf_handle *h, int *tile_rows, int *z_chunk) {
   return PF_OK;
 }
 
+int pf_adjoint_release(pf_handle *h) {
+  if (!h) return PF_ERR_INVALID;
+  hipSetDevice(h->d.device);
+  kept_blocks().drop(h, false);
+  return PF_OK;
+}
+
 int pf_list_lengths(pf_handle *h, int64_t *sweep_listed, int64_t *diffusion_listed) {
   if (!h) return PF_ERR_INVALID;
   hipSetDevice(h->d.device);
@@ -1512,7 +1540,7 @@ int pf_setup_construct(pf_handle *h, const double *seeds, int G, double reductio
   hipSetDevice(h->d.device);
   const int K = h->d.depth, P = h->d.nphase;
   double *dseeds = nullptr;
-  HIPCHK(h, hipMalloc(&dseeds, sizeof(double) * 3 * G));
+  HIPCHK(h, device_malloc(&dseeds, sizeof(double) * 3 * G));
   hipError_t e = hipMemcpyAsync(dseeds, seeds, sizeof(double) * 3 * G, hipMemcpyHostToDevice,
                                 h->stream);
   double *phi = static_cast<double *>(h->phi[0]), *pf = static_cast<double *>(h->pfrac);
@@ -1616,9 +1644,9 @@ int pf_setup_nucleate(pf_handle *h, int n_nuclei, float radius, const double *nu
     if (mark) hipFree(mark);
     if (best) hipFree(best);
   };
-  hipError_t e = hipMalloc(&flag, N * 4);
-  if (e == hipSuccess) e = hipMalloc(&mark, N);
-  if (e == hipSuccess) e = hipMalloc(&best, (size_t(nchunk) + 1) * 8);
+  hipError_t e = device_malloc(&flag, N * 4);
+  if (e == hipSuccess) e = device_malloc(&mark, N);
+  if (e == hipSuccess) e = device_malloc(&best, (size_t(nchunk) + 1) * 8);
   if (e != hipSuccess) {
     cleanup();
     return fail(h, PF_ERR_OOM, "nucleation scratch allocation failed");
@@ -1918,22 +1946,11 @@ int handle_diffuse_io(pf_handle *h, const double *cin, double *cout) {
 }
 void handle_count_substeps(pf_handle *h, int n) { h->csub[0] += uint32_t(n); }
 bool handle_use_direct(const pf_handle *h) { return use_direct(h, h->NF); }
-void handle_adjoint_release(pf_handle *h) {
-  if (h->adj_block) hipFree(h->adj_block);
-  h->adj_block = nullptr;
-  h->adj_bytes = 0;
+void *handle_adjoint_take(pf_handle *h, size_t bytes) {
+  return kept_blocks().take(h, h->d.device, bytes);
 }
-size_t handle_adjoint_kept(const pf_handle *h) { return h->adj_bytes; }
-void *handle_adjoint_block(pf_handle *h, size_t bytes) {
-  if (h->adj_bytes >= bytes) return h->adj_block;
-  handle_adjoint_release(h);
-  if (hipMalloc(&h->adj_block, bytes) != hipSuccess) {
-    h->adj_block = nullptr;
-    return nullptr;
-  }
-  h->adj_bytes = bytes;
-  return h->adj_block;
-}
+void handle_adjoint_done(pf_handle *h, size_t most) { kept_blocks().done(h, most); }
+size_t handle_adjoint_idle(const pf_handle *h) { return kept_blocks().idle(h->d.device); }
 void handle_state_changed(pf_handle *h) {
   h->flag_valid = false;
   h->unit_valid = false;

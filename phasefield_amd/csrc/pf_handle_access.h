@@ -40,9 +40,10 @@ int handle_diffuse_io(pf_handle *h, const double *cin, double *cout);
 void handle_count_substeps(pf_handle *h, int n);
 // whether this handle's single sub-steps run as one launch of the direct kernel
 bool handle_use_direct(const pf_handle *h);
-// Device memory of the adjoint, kept between runs and freed with the handle: a block of at least
-// `bytes`, the kept one when it is large enough (null: out of memory).
-void *handle_adjoint_block(pf_handle *h, size_t bytes);
-// bytes of the kept block, and giving it back
-size_t handle_adjoint_kept(const pf_handle *h);
-void handle_adjoint_release(pf_handle *h);
+// Device memory of the adjoint, one block per handle that is kept between runs (pf_kept_blocks.h): take
+// a block of at least `bytes` (null: out of memory), end the run's use of it (a block of more than `most`
+// bytes goes back), and the bytes that are kept idle on the handle's device, by any handle, which a
+// `take` gets if it needs them.
+void *handle_adjoint_take(pf_handle *h, size_t bytes);
+void handle_adjoint_done(pf_handle *h, size_t most);
+size_t handle_adjoint_idle(const pf_handle *h);
