@@ -12,9 +12,11 @@ by stream synchronisation.
 
 Roofline of the dominant kernel, the plane-marching diffusion kernel (about 80 % of a step): the
 bytes it must move per launch (every cell's stored concentration read once and written once: FP64
-8 + 8 B, mixed 4 + 1 B each way) over its mean launch time from HIP event pairs around a sample of
-its launches inside the timed region, on the stream it runs on (domains that do not take it: the same
-bytes over the sub-step, named by its kernel).  `substep` adds the listed pass
+8 + 8 B, mixed 4.5 B each way) over its mean launch time from HIP event pairs around a sample of
+its launches inside the timed region, on the stream it runs on.  Domains that do not take it name the
+kernel that the library runs: the one-launch kernel with the same bytes over the sub-step, tiles
+(several sub-steps of a plane per launch, in LDS) with their time per sub-step and no bandwidth.
+`substep` adds the listed pass
 (the cells next to a phase boundary, full formula) with the list length read from the device, and
 the gaps between the two launches.  `model_8d` states the same run in the compulsory-traffic model
 of the scope document (every cell reads value_phase; 24 / 32 B per cell per sub-step).
@@ -126,16 +128,61 @@ def measured_traffic(workload: str) -> dict:
     return {}
 
 
-def substep_kernel_name(is_mixed: bool, nphase: int, dims: int) -> str:
-    """The kernel of a sub-step that is not the marching kernel's (2D: several sub-steps a launch)."""
-    kernel = "diffuse_tile_kernel" if dims == 2 else "diffuse_direct_kernel"
-    return f"{kernel}<{'FormMixed' if is_mixed else 'FormF64'}, {nphase}>"
-
-
 def march_kernel_name(mixed: bool, nphase: int, noflux: bool, rows: int) -> str:
     form = "FormMixed" if mixed else "FormF64"
     return (f"diffuse_bulk_march_kernel<{form}, {nphase}, 6, {'true' if noflux else 'false'}, "
             f"{rows}, {4 if mixed else 2}, 1>")
+
+
+def rate(nbytes: float, ms: float, count: int) -> tuple[float | None, float | None]:
+    """(GB/s, fraction of the HBM peak) of `count` launches of `nbytes` each in `ms`; none timed: None."""
+    if not count or ms <= 0.0:
+        return None, None
+    gbs = nbytes * count / (ms * 1e-3) / 1e9
+    return round(gbs, 1), round(gbs / HBM_PEAK_GBS, 4)
+
+
+def mean_us(ms: float, count: int) -> float | None:
+    return round(ms / count * 1e3, 2) if count else None
+
+
+def rooflines(is_mixed: bool, nphase: int, noflux: bool, ncell: int, t: dict, kernel: str, substeps: int,
+              rows: int, zchunk: int, diff_listed: int, traffic: dict | None) -> tuple[dict, dict]:
+    """The roofline of the dominant kernel, and the whole sub-step, from the timed launches `t` (kind ->
+    (ms, count)) and the bulk kernel that the library ran, with the sub-steps of one launch of it.
+
+    The marching kernel has launches of its own, beside the listed pass.  The one-launch kernel is the
+    sub-step.  A tile launch takes its cells through several sub-steps in LDS: what it moves belongs to
+    no one of them, so only its time per sub-step is given."""
+    bpc = march_bytes_per_cell(is_mixed)
+    march = bool(t["march"][1])
+    per_substep = march or substeps == 1
+    ms, count = t["march"] if march else t["sub"]
+    name = (march_kernel_name(is_mixed, nphase, noflux, rows) if march else
+            f"{kernel}<{'FormMixed' if is_mixed else 'FormF64'}, {nphase}>")
+    achieved, frac = rate(ncell * bpc, ms, count) if per_substep else (None, None)
+    # the summary records each profiled tile shape's bytes by kernel name; the tuner's pick on this
+    # device selects one (none when it picked a shape the summary did not profile)
+    measured = traffic.get("march", {}).get(name) if traffic and not traffic.get("stale") else None
+    roofline = {"bound": "hbm" if per_substep else "latency", "achieved": achieved, "peak": HBM_PEAK_GBS,
+                "unit": "GB/s", "frac": frac, "traffic": measured, "kernel": name, "tile_rows": rows,
+                "z_chunk": zchunk, "bytes_per_cell": bpc if per_substep else None,
+                "cells_per_launch": ncell, "substeps_per_launch": substeps,
+                "launch_us" if per_substep else "substep_us": mean_us(ms, count),
+                "launches_timed" if per_substep else "substeps_timed": count,
+                "traffic_source": (f"{traffic.get('file')} (kernel sources {traffic.get('sources')}"
+                                   f"{', stale: not used' if traffic.get('stale') else ''})"
+                                   if traffic else None),
+                "traffic_frac": rate(measured, ms, count)[1] if measured else None}
+    # a listed pass adds its own traffic; in one launch the listed cells are among the bytes above
+    lbpc = listed_bytes_per_cell(is_mixed, nphase)
+    nbytes = ncell * bpc + (0 if kernel == "diffuse_direct_kernel" else diff_listed * lbpc)
+    ms, count = t["sub"]
+    gbs, frac = rate(nbytes, ms, count) if per_substep else (None, None)
+    return roofline, {"us": mean_us(ms, count), "launches_timed": count, "listed_cells": diff_listed,
+                      "listed_fraction": round(diff_listed / ncell, 6),
+                      "bytes": nbytes if per_substep else None, "listed_bytes_per_cell": lbpc,
+                      "achieved_gbs": gbs, "frac": frac}
 
 
 def timed_run(dom, model, steps: int, warmup: int):
@@ -505,50 +552,21 @@ def main() -> int:
         sweep_listed, diff_listed = dom.list_lengths()
         rows, zc = dom.march_shape()
         st = dom.reduce()
-        sub_us = t["sub"][0] / max(t["sub"][1], 1) * 1e3
-        # domains whose whole sub-step is one launch (or several sub-steps of a plane) have no
-        # marching launches: the roofline is the sub-step's then
-        dominant = "march" if t["march"][1] else "sub"
-        march_us = t[dominant][0] / max(t[dominant][1], 1) * 1e3
+        roofline, substep = rooflines(is_mixed, d.nphase, noflux, N, t, *dom.substep_kernel(), rows, zc,
+                                      diff_listed, traffic)
         sweep_us = t["sweep"][0] / t["sweep"][1] * 1e3
-        bpc = march_bytes_per_cell(is_mixed)
-        achieved = N * bpc / (max(march_us, 1e-3) * 1e-6) / 1e9
-        kname = (march_kernel_name(is_mixed, d.nphase, noflux, rows) if dominant == "march" else
-                 substep_kernel_name(is_mixed, d.nphase, 2 if d.nz == 1 else 3))
-        # the summary records each profiled tile shape's bytes by kernel name; the tuner's pick
-        # on this device selects one (none when it picked a shape the summary did not profile)
-        measured = (traffic.get("march", {}).get(kname)
-                    if traffic and not traffic.get("stale") else None)
-        lbpc = listed_bytes_per_cell(is_mixed, d.nphase)
-        sub_bytes = N * bpc + diff_listed * lbpc
         res[name] = {
             "wall": wall, "ms_per_step": wall / args.steps * 1e3, "value": N * args.steps / wall / 1e9,
             "stats": st,
-            "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
-                         "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                         "traffic": measured,
-                         "kernel": kname, "tile_rows": rows, "z_chunk": zc,
-                         "bytes_per_cell": bpc, "cells_per_launch": N,
-                         "launch_us": round(march_us, 2), "launches_timed": t[dominant][1],
-                         "traffic_source": (f"{traffic.get('file')} (kernel sources "
-                                            f"{traffic.get('sources')}"
-                                            f"{', stale: not used' if traffic.get('stale') else ''})"
-                                            if traffic else None),
-                         "traffic_frac": (round(measured / (march_us * 1e-6) / 1e9 / HBM_PEAK_GBS, 4)
-                                          if measured else None)},
-            "substep": {"us": round(sub_us, 2), "launches_timed": t["sub"][1],
-                        "listed_cells": diff_listed,
-                        "listed_fraction": round(diff_listed / N, 6),
-                        "bytes": sub_bytes, "listed_bytes_per_cell": lbpc,
-                        "achieved_gbs": round(sub_bytes / (max(sub_us, 1e-3) * 1e-6) / 1e9, 1),
-                        "frac": round(sub_bytes / (max(sub_us, 1e-3) * 1e-6) / 1e9 / HBM_PEAK_GBS, 4)},
+            "roofline": roofline,
+            "substep": substep,
             "sweep": {"us": round(sweep_us, 1), "listed_cells": sweep_listed,
                       "listed_fraction": round(sweep_listed / N, 6)},
         }
-        log(f"{name}: {res[name]['ms_per_step']:.2f} ms/step, "
-            f"{'march' if dominant == 'march' else 'one launch'} {march_us:.1f} us "
-            f"({achieved:.0f} GB/s), sub-step {sub_us:.1f} us ({res[name]['substep']['frac']:.3f} of "
-            f"peak, {diff_listed} listed), sweep {sweep_us:.0f} us ({sweep_listed} listed)")
+        log(f"{name}: {res[name]['ms_per_step']:.2f} ms/step, {roofline['kernel']} "
+            f"{roofline.get('launch_us')} us ({roofline['achieved']} GB/s), sub-step {substep['us']} us "
+            f"({substep['frac']} of peak, {diff_listed} listed), sweep {sweep_us:.0f} us "
+            f"({sweep_listed} listed)")
 
     mx = res["mixed"]
     n_sub = p0.n_sub[0]
@@ -581,7 +599,8 @@ def main() -> int:
                        "dtype": "f64", "roofline": f64["roofline"], "substep": f64["substep"],
                        "sweep": f64["sweep"], "model_8d": f64["model_8d"]}
         out["mixed_over_fp64"] = round(mx["value"] / f64["value"], 4)
-        out["march_fp64_over_mixed"] = round(f64["roofline"]["launch_us"] / max(mx["roofline"]["launch_us"], 1e-3), 4)
+        us = [r["roofline"].get("launch_us") for r in (f64, mx)]
+        out["march_fp64_over_mixed"] = round(us[0] / us[1], 4) if all(us) else None
         done = args.warmup + args.steps
         if args.accuracy_steps > done:
             log(f"accuracy: both forms to step {args.accuracy_steps}")

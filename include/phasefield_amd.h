@@ -148,6 +148,9 @@ int pf_list_lengths(pf_handle *h, int64_t *sweep_listed, int64_t *diffusion_list
 /* Tile rows and z-chunk of the plane-marching diffusion kernel on this handle (picked by timing the
  * candidate shapes at the first sub-step); 0, 0 before that or when that kernel is not in use. */
 int pf_march_shape(const pf_handle *h, int *tile_rows, int *z_chunk);
+/* Name of the kernel that updated the bulk cells in the last sub-steps, and how many sub-steps its last
+ * launch did (planes on tiles: several); NULL and 0 before the first.  The string is static. */
+const char *pf_substep_kernel(const pf_handle *h, int *substeps);
 /* Size in bytes of one checkpoint of this handle.  save/restore copy the whole state, the mixed
  * form's sub-step counters and the grain-code tables to / from host memory of that size; restore
  * rejects a blob whose header names another domain shape, form or size. */

@@ -212,6 +212,12 @@ class Domain:
         _check(lib().pf_march_shape(self._h, C.byref(a), C.byref(b)), self._h, "march shape")
         return a.value, b.value
 
+    def substep_kernel(self) -> tuple[str | None, int]:
+        """(bulk kernel of the last sub-steps, sub-steps of its last launch); (None, 0) before the first."""
+        k = C.c_int()
+        name = lib().pf_substep_kernel(self._h, C.byref(k))
+        return name.decode() if name else None, k.value
+
     # --- checkpoints -------------------------------------------------------------------------
     def checkpoint(self) -> bytes:
         n = C.c_size_t()

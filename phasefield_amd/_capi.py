@@ -89,6 +89,7 @@ SIGNATURES = {
     "pf_dump_wait": (_I, [_H]),
     "pf_kernel_timing": (_I, [_H, _I, C.POINTER(_D), C.POINTER(C.c_int64)]),
     "pf_kernel_timing_reset": (_I, [_H, _I]),
+    "pf_substep_kernel": (C.c_char_p, [_H, C.POINTER(_I)]),
     "pf_list_lengths": (_I, [_H, C.POINTER(C.c_int64), C.POINTER(C.c_int64)]),
     "pf_march_shape": (_I, [_H, C.POINTER(_I), C.POINTER(_I)]),
     "pf_checkpoint_size": (_I, [_H, C.POINTER(C.c_size_t)]),

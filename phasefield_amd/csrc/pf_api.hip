@@ -86,6 +86,8 @@ struct pf_handle {
   bool diff_march = true;    // ... in its plane-marching form
   int march_by = 0;          // its tile rows and z-chunk, picked by timing at first use
   int march_zc = 0;
+  const char *bulk_kernel = nullptr;  // kernel and sub-steps of the last sub-step launch (bulk cells)
+  int bulk_steps = 0;
   bool flip = false;         // direction of the direct kernel's next pass (alternates)
   int *list_len = nullptr;   // [0]: cells the last sweep listed, [1]: cells the diffusion lists
   int *ccount = nullptr;     // pair lists: listed cells per list block ([nblocks + 1])
@@ -618,7 +620,12 @@ hipError_t launch_diffuse_io(pf_handle *h, const DiffConsts<typename F::A> &dc,
                              const typename F::C *cin, typename F::C *cout) {
   using T = typename F::T;
   const T *pf = static_cast<const T *>(h->pfrac);
+  auto note = [h](const char *kernel) {
+    h->bulk_kernel = kernel;
+    h->bulk_steps = 1;
+  };
   if (h->diff_variant == 1) {
+    note("diffuse_kernel");
     const DiffGeom g = diff_geom(h, kDiffTY, 2048, 16);
     hipLaunchKernelGGL((diffuse_kernel<F, P, NF, NOF, kDiffTY>), dim3(g.nblocks),
                        dim3(64, kDiffTY + 3), 0, h->stream, cin, cout, pf, dc, h->d.nx, h->d.ny,
@@ -632,6 +639,7 @@ hipError_t launch_diffuse_io(pf_handle *h, const DiffConsts<typename F::A> &dc,
     if (h->diff_split && h->list_stale) build_list<F>(h, NF);
     if constexpr (NF == 6) {
       if (use_direct(h, NF)) {
+        note("diffuse_direct_kernel");
         h->flip = !h->flip;  // the next sub-step starts where this one ends
         return launch_direct<F, P, NOF>(h->stream, cin, cout, pf, h->packed, h->glist,
                                         h->gblock + list_blocks(h->N), dc, h->d.nx, h->d.ny, h->d.nz,
@@ -642,6 +650,7 @@ hipError_t launch_diffuse_io(pf_handle *h, const DiffConsts<typename F::A> &dc,
       constexpr int BY = decltype(by)::value;
       constexpr bool SPLIT = decltype(split)::value;
       // z-chunks of ~16 planes: the measured optimum at 512^3 (4 tile rows, 8192+ workgroups)
+      note("diffuse_bulk_kernel");
       const DiffGeom g = diff_geom(h, BY, 131072 / BY, 8);
       hipLaunchKernelGGL((diffuse_bulk_kernel<F, P, NF, NOF, BY, SPLIT>), dim3(g.nblocks),
                          dim3(64, BY), 0, h->stream, cin, cout, pf, h->flag, dc, h->d.nx, h->d.ny,
@@ -651,10 +660,11 @@ hipError_t launch_diffuse_io(pf_handle *h, const DiffConsts<typename F::A> &dc,
       constexpr bool SPLIT = decltype(split)::value;
       // below ~64M cells the storage-order kernel measured faster (caches hold more of the domain)
       const int by = h->diff_by >= 0 ? h->diff_by : (h->N < (1L << 26) ? 0 : 4);
-      if (by == 0)
+      if (by == 0) {
+        note("diffuse_linear_kernel");
         hipLaunchKernelGGL((diffuse_linear_kernel<F, P, NF, NOF, SPLIT>), dim3(nb), dim3(256), 0,
                            h->stream, cin, cout, pf, h->flag, dc, h->d.nx, h->d.ny, h->d.nz);
-      else if (by == 16)
+      } else if (by == 16)
         go(std::integral_constant<int, 16>(), split);
       else if (by == 8)
         go(std::integral_constant<int, 8>(), split);
@@ -662,12 +672,14 @@ hipError_t launch_diffuse_io(pf_handle *h, const DiffConsts<typename F::A> &dc,
         go(std::integral_constant<int, 4>(), split);
     };
     if (march) {
+      note("diffuse_bulk_march_kernel");
       // kind 2: this launch alone, on sampled sub-steps once the shape is picked
       Timer t(h, 2, h->time_march && h->march_by != 0 ? 1 : 0);
       const hipError_t e = launch_march<F, P, NF, NOF>(h, dc, cin, cout);
       if (e != hipSuccess) return e;
     } else if (h->diff_split && h->diff_vec && h->d.nx % V == 0 &&
                (h->diff_by < 0 || h->diff_by == 4)) {
+      note("diffuse_bulk_vec_kernel");
       const DiffGeom g = diff_geom(h, 4, 131072 / 4, 8, 64 * V);
       hipLaunchKernelGGL((diffuse_bulk_vec_kernel<F, P, NF, NOF, 4, V>), dim3(g.nblocks),
                          dim3(64, 4), 0, h->stream, cin, cout, h->flag, dc, h->d.nx, h->d.ny,
@@ -736,6 +748,8 @@ hipError_t launch_tile(pf_handle *h, int s, const DiffConsts<typename F::A> &dc,
                      h->stream, static_cast<const C *>(h->conc[s][a]),
                      static_cast<C *>(h->conc[s][b]), static_cast<const T *>(h->pfrac), h->flag, dc,
                      g, h->N, h->csub[s], s);
+  h->bulk_kernel = "diffuse_tile_kernel";
+  h->bulk_steps = g.steps;
   h->ccur[s] = b;
   h->csub[s] += uint32_t(g.steps);
   return hipGetLastError();
@@ -1377,6 +1391,11 @@ int pf_march_shape(const pf_handle *h, int *tile_rows, int *z_chunk) {
   if (!h) return PF_ERR_INVALID;
   handle_march_shape(h, tile_rows, z_chunk);
   return PF_OK;
+}
+
+const char *pf_substep_kernel(const pf_handle *h, int *substeps) {
+  if (substeps) *substeps = h ? h->bulk_steps : 0;
+  return h ? h->bulk_kernel : nullptr;
 }
 
 int pf_adjoint_release(pf_handle *h) {

@@ -228,3 +228,27 @@ def test_accelerator_calls_against_the_oracle(shape, loops, params):  # noqa: F8
                                                q.dx, stream)
     assert rc == 0, lib().pf_last_error(None)
     assert np.flatnonzero(dconc.cpu().numpy() != want)[:20].tolist() == []
+
+
+@pytest.mark.parametrize("shape,pins,kernel,substeps", [
+    ((64, 48, 1), {}, "diffuse_tile_kernel", 6),  # 20 sub-steps as 7 + 7 + 6
+    ((64, 20, 12), {}, "diffuse_direct_kernel", 1),
+    ((300, 1, 300), {}, "diffuse_bulk_march_kernel", 1),
+    ((64, 20, 12), {"PFAMD_DIFF_DIRECT": "0"}, "diffuse_bulk_march_kernel", 1),
+    ((33, 20, 12), {"PFAMD_DIFF_DIRECT": "0"}, "diffuse_linear_kernel", 1),
+    ((64, 20, 12), {"PFAMD_DIFF_MARCH": "0"}, "diffuse_bulk_vec_kernel", 1),
+    ((64, 20, 12), {"PFAMD_DIFF_VEC": "0", "PFAMD_DIFF_BY": "4"}, "diffuse_bulk_kernel", 1),
+    ((64, 20, 12), {"PFAMD_DIFF_KERNEL": "lds"}, "diffuse_kernel", 1)])
+def test_substep_kernel_is_named(monkeypatch, shape, pins, kernel, substeps, params):  # noqa: F811
+    print(f"[gpu] sub-step kernel of {shape} {pins}", flush=True)
+    for k, v in pins.items():
+        monkeypatch.setenv(k, v)
+    q = PfParams.from_buffer_copy(params)
+    q.dims = 3 - (shape[2] == 1) - (shape[1] == 1)
+    g = Domain(*shape, depth=4)
+    g.set_params(q)
+    g.upload(*sub.sparse_state(np.random.default_rng(45), *shape, 2))
+    assert g.substep_kernel() == (None, 0)
+    g.diffuse(0, 20, q.dt_d[0])
+    assert g.substep_kernel() == (kernel, substeps)
+    g.close()
