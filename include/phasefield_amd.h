@@ -136,14 +136,19 @@ int pf_reduce(pf_handle *h, pf_stats *out);
 int pf_synchronize(pf_handle *h);
 /* Device time in ms of the dominant kernel launches since the last reset, and how many launches
  * it covers (HIP event pairs on the handle's stream); kind 0 = diffusion sub-step (one pair around
- * each batch of back-to-back sub-steps, leaving out a batch's first sub-step, which also classifies
- * bulk cells), 1 = phase-field sweep, 2 = the plane-marching bulk kernel alone (one pair around
- * every eighth of those sub-steps' bulk launches). */
+ * each batch of back-to-back sub-steps, leaving out a batch's first launch, which also classifies
+ * bulk cells; counted in sub-steps, of which a launch on planes does up to 12), 1 = phase-field
+ * sweep, 2 = the plane-marching bulk kernel alone (one pair around every eighth of those sub-steps'
+ * bulk launches). */
 int pf_kernel_timing(pf_handle *h, int kind, double *total_ms, int64_t *launches);
 int pf_kernel_timing_reset(pf_handle *h, int enable);
 /* Lengths of the per-sweep cell lists the step works through (synchronises): the cells the last
- * phase-field sweep updated with the full formula (the rest were copied), and the cells the
- * diffusion sub-steps update with the full formula (the rest take the bulk update). */
+ * phase-field sweep updated with the full formula (the rest were copied), and the cells that the
+ * listed pass of the diffusion sub-steps updates with the full formula: those that are not bulk cells
+ * of the most common bulk phase, or, with the kernels that tell the phases apart, of any bulk phase.
+ * The one-launch and tile kernels (pf_substep_kernel) tell them apart and have no listed pass; there the
+ * count is that of the marching kernel where rows would suit it, an upper bound of the cells that get
+ * the full formula. */
 int pf_list_lengths(pf_handle *h, int64_t *sweep_listed, int64_t *diffusion_listed);
 /* Tile rows and z-chunk of the plane-marching diffusion kernel on this handle (picked by timing the
  * candidate shapes at the first sub-step); 0, 0 before that or when that kernel is not in use. */
