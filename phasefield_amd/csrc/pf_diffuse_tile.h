@@ -10,7 +10,6 @@ namespace pfamd {
 // 1.59 instead of 1.42 us (256^2 FP64): it is a chain of LDS and FP64 latencies, hidden by wavefronts.
 constexpr int kTileNT = 1024;  // threads of a workgroup
 constexpr int kTileV = 2;      // cells per thread: a tile and its halo hold at most kTileNT * kTileV
-constexpr int kTileG = 1;      // listed cells per thread, held in registers
 
 // Geometry of a launch of up to `left` sub-steps on nz planes of nx x ny cells; false when single
 // sub-steps are faster.  pin: tile and sub-steps to use instead (pin[2] == 0: none).

@@ -10,41 +10,51 @@
 // A bulk cell (flag p) is owned by a thread and takes the reduced update.  The listed cells (flag 0)
 // are compacted per tile; each is an entry of one thread, which keeps the cell's face weights and
 // partition constants in registers for all sub-steps of the launch and publishes the cell's
-// partition in LDS for the entries next to it.  A tile with more listed cells than entries takes
-// them from memory instead (the full formula, every sub-step).
+// partition in LDS for the entries next to it.  A tile with more listed cells than threads gives every
+// thread two: its second instance of the sub-steps is held to the registers that the first needs (a
+// few of its values are spilled; 116 instead of 96 VGPRs cost every FP64 step 3 % in turn with other
+// domains' kernels).  Per sub-step, one domain, every cell listed: from memory (the full formula each
+// time, as it was) / two entries / single sub-steps:
+//   256^2 FP64        6.98 / 2.85 / 8.1 us      1000 x 600 FP64     27.8 / 14.9 / 20.4 us
+//   256^2 mixed       4.45 / 3.12 / 8.7         1000 x 600 mixed    16.3 / 12.9 / 14.0
+//   256^2, 3 phases   8.52 / 3.29 / 9.0         1200^2 FP64         54.2 / 29.0 / 35.6
+// The third phase's terms are 0 * (0 - 0) where no entry of a wavefront and none of its neighbours has
+// that phase, and are left out there (256^2 accelerator call 322 -> 307 us).
 //
 // A one-cell-thick domain whose stencil has six faces (the accelerator calls) runs here as well: its
 // z faces join a cell to itself and carry no flux, only the NaN of a partition that is not finite
 // (SELF_Z; an infinite bulk cell becomes NaN without them).
 #include "pf_diffuse_tile.h"
 
+#include <type_traits>
+
 namespace pfamd {
 
 template <class F, int P, bool SELF_Z>
-__global__ __launch_bounds__(kTileNT) void diffuse_tile_kernel(
+__global__ __launch_bounds__(kTileNT, P == 2 ? (F::kMixed ? 8 : 5) : 4) void diffuse_tile_kernel(
     const typename F::C *__restrict__ cin, typename F::C *__restrict__ cout,
     const typename F::T *__restrict__ pfrac, const uint8_t *__restrict__ flag,
     const DiffConsts<typename F::A> dc, const TileGeom geo, const long ncell, const uint32_t k0,
     const int solute) {
   using A = typename F::A;
-  constexpr int NF = 4, NT = kTileNT, V = kTileV, G = kTileG;
-  constexpr int CELLS = NT * V, SLOTS = NT * G;
-  constexpr int EXTRA = SLOTS * P > CELLS ? SLOTS * P : CELLS;
-  constexpr int NONE = CELLS + EXTRA;  // the partition of an absent phase
+  constexpr int NF = 4, NT = kTileNT, V = kTileV, CELLS = NT * V;
+  constexpr int NONE = CELLS + CELLS * P;  // the partition of an absent phase
   static_assert(NONE < 65535, "16-bit element indices");
-  static_assert(V <= 8 && G * P <= 32, "packed codes and presence bits");
-  __shared__ A L[NONE + 1];            // the cells' values; behind them the entries' partitions (or,
-                                       // in a dense tile, the listed cells' new values); 0
+  static_assert(V <= 8 && V * P <= 32, "packed codes and presence bits");
+  __shared__ A L[NONE + 1];            // the cells' values; behind them the entries' partitions; 0
   __shared__ uint16_t slot_of[CELLS];  // a listed cell's entry, 0xffff for the others
   __shared__ uint16_t list[CELLS];     // the listed cells
   __shared__ uint8_t codes[F::kMixed ? CELLS : 1];
   __shared__ int counter;
   const int t = threadIdx.x;
   const int nx = geo.nx, ny = geo.ny, S = geo.steps;
-  // workgroup b runs on XCD b % 8: each XCD takes a contiguous range of tiles
-  const int b = blockIdx.x;
-  const int per = geo.nblocks >> 3, rem = geo.nblocks & 7, xcd = b & 7;
-  const int logical = xcd * per + (xcd < rem ? xcd : rem) + (b >> 3);
+  // Workgroup b runs on XCD b % 8: of every 256 tiles in a row (one per compute unit) each XCD takes a
+  // contiguous eighth, so that neighbouring tiles share its L2 and tiles full of listed cells, which
+  // lie side by side, spread over the XCDs (1000 x 600 FP64, 30 % of the plane listed: 14.5 us per
+  // sub-step with eighths of all tiles, 7.7 with these).
+  const int b = blockIdx.x, group = b & ~255;
+  const int m = min(256, geo.nblocks - group), xcd = b & 7;
+  const int logical = group + xcd * (m >> 3) + min(xcd, m & 7) + ((b & 255) >> 3);
   const int tx = logical % geo.nbx, tyz = logical / geo.nbx;
   const int ty = tyz % geo.nby;
   const uint32_t plane0 = uint32_t(nx) * uint32_t(ny) * uint32_t(tyz / geo.nby);
@@ -183,7 +193,9 @@ __global__ __launch_bounds__(kTileNT) void diffuse_tile_kernel(
     o.gn[3] = gy == ny - 1 ? g + unx - plane : g + unx;
   };
 
-  if (ng <= SLOTS) {
+  // the sub-steps, with up to G listed cells per thread
+  auto run = [&](auto entries) {
+    constexpr int G = decltype(entries)::value;
     A w[G][NF * P], t1[G][P], t2[G][P], cp[G][P], sc[G];
     int sdepth[G];
     // saddr: a neighbour's partition in L by face and phase, two places per word.  A bulk neighbour's
@@ -193,13 +205,17 @@ __global__ __launch_bounds__(kTileNT) void diffuse_tile_kernel(
     uint32_t saddr[G][NF * P / 2], sgi[G], present = 0;
     CompCode sq[G];
     // partition_cell of an entry's value (the division by t1 = 1 of a unit cell changes nothing)
+    // whether an entry of the wavefront or a neighbour has the third phase (or its D is not finite)
+    bool third = true;
     auto partition = [&](int j) {
 #pragma unroll
       for (int p = 0; p < P; ++p) {
+        if (p == 2 && !third) continue;
         const A v = (sc[j] - t2[j][p]) / t1[j][p];
         cp[j][p] = ((present >> (j * P + p)) & 1u) ? v : A(0);
       }
     };
+    bool has = false;
 #pragma unroll
     for (int j = 0; j < G; ++j) {
       const int slot = t + j * NT;
@@ -229,6 +245,11 @@ __global__ __launch_bounds__(kTileNT) void diffuse_tile_kernel(
         for (int f = 0; f < NF; ++f)
 #pragma unroll
           for (int p = 0; p < P; ++p) phn[f][p] = A(pfrac[long(o.gn[f]) * P + p]);
+        if constexpr (P == 3) {
+          has = has || !(ph[2] == A(0));
+#pragma unroll
+          for (int f = 0; f < NF; ++f) has = has || !(phn[f][2] == A(0));
+        }
         // (a cell of the outermost layer is never updated; only its partition is read)
 #pragma unroll
         for (int f = 0; f < NF; ++f) {
@@ -266,6 +287,7 @@ __global__ __launch_bounds__(kTileNT) void diffuse_tile_kernel(
         for (int p = 0; p < P; ++p) L[CELLS + slot * P + p] = cp[j][p];
       }
     }
+    if constexpr (P == 3) third = __any(has) || !(dc.D[2] * A(0) == A(0));
     __syncthreads();
     const int waves_first = t & ~63;  // entries of this wavefront: waves_first + j * NT and on
     for (int s = 1; s <= S; ++s) {
@@ -280,6 +302,7 @@ __global__ __launch_bounds__(kTileNT) void diffuse_tile_kernel(
         for (int f = 0; f < NF; ++f)
 #pragma unroll
           for (int p = 0; p < P; ++p) {
+            if (p == 2 && !third) continue;  // 0 * (0 - 0)
             const int q = f * P + p;
             const uint32_t a = (saddr[j][q >> 1] >> (16 * (q & 1))) & 0xffffu;
             const A term = w[j][q] * (L[a] - cp[j][p]);
@@ -314,53 +337,9 @@ __global__ __launch_bounds__(kTileNT) void diffuse_tile_kernel(
       for (int j = 0; j < G; ++j)
         if (sdepth[j] > 0) codes[list[t + j * NT]] = uint8_t(uint32_t(sq[j]) & 15u);
     }
-  } else {
-    // more listed cells than entries: the new values are kept behind the cells until every thread
-    // has read
-    for (int s = 1; s <= S; ++s) {
-      const uint32_t key = key_of(s);
-      bulk_step(s, key);
-      for (int i = t; i < ng; i += NT) {
-        const int idx = list[i];
-        Cell o;
-        locate(idx, o);
-        A v = L[idx];
-        if (o.depth >= s) {
-          StencilLoad<F, P, NF> st;
-          st.me.c = typename F::C(v);
-#pragma unroll
-          for (int p = 0; p < P; ++p) st.me.ph[p] = pfrac[long(o.g) * P + p];
-          A z = A(0);
-          if constexpr (SELF_Z) {  // (before the neighbours are loaded: registers)
-            CellPF<A> me;
-            partition_cell<F, P>(st.me, dc, me);
-            z = self_z(me.c);
-            asm volatile("" : "+v"(z));
-          }
-#pragma unroll
-          for (int f = 0; f < NF; ++f) {
-            st.nb[f].c = typename F::C(L[idx + o.off[f]]);
-#pragma unroll
-            for (int p = 0; p < P; ++p) st.nb[f].ph[p] = pfrac[long(o.gn[f]) * P + p];
-          }
-          A del = stencil_del<F, P, NF>(st, dc);
-          if constexpr (SELF_Z) del += z;
-          if constexpr (F::kMixed) {
-            CompCode qo;
-            v = mixed_step(v, del, comp_unpack(codes[idx]), comp_hash(o.g, key), qo);
-            codes[idx] = uint8_t(uint32_t(qo) & 15u);
-          } else {
-            v = v + del;
-          }
-        }
-        L[CELLS + i] = v;
-      }
-      __syncthreads();
-      bulk_write(s);
-      for (int i = t; i < ng; i += NT) L[list[i]] = L[CELLS + i];
-      __syncthreads();
-    }
-  }
+  };
+  if (__builtin_expect(ng <= NT, 1)) run(std::integral_constant<int, 1>());
+  else run(std::integral_constant<int, V>());
 
 #pragma unroll
   for (int k = 0; k < V; ++k)
