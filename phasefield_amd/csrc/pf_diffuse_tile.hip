@@ -11,13 +11,14 @@
 // are compacted per tile; each is an entry of one thread, which keeps the cell's face weights and
 // partition constants in registers for all sub-steps of the launch and publishes the cell's
 // partition in LDS for the entries next to it.  A tile with more listed cells than threads gives every
-// thread two: its second instance of the sub-steps is held to the registers that the first needs (a
-// few of its values are spilled; 116 instead of 96 VGPRs cost every FP64 step 3 % in turn with other
-// domains' kernels).  Per sub-step, one domain, every cell listed: from memory (the full formula each
-// time, as it was) / two entries / single sub-steps:
-//   256^2 FP64        6.98 / 2.85 / 8.1 us      1000 x 600 FP64     27.8 / 14.9 / 20.4 us
-//   256^2 mixed       4.45 / 3.12 / 8.7         1000 x 600 mixed    16.3 / 12.9 / 14.0
-//   256^2, 3 phases   8.52 / 3.29 / 9.0         1200^2 FP64         54.2 / 29.0 / 35.6
+// thread two.  Two of three phases would not fit the registers: where a tile that full has the third
+// phase it takes the full formula from memory, every sub-step.  The two-phase FP64 kernel is held to 96
+// registers (a few values of the second instance are spilled): at 116 every step took 3 % longer in turn
+// with other domains' kernels.  Per sub-step, one domain, every cell listed, from memory (as it was) /
+// with two entries / single sub-steps:
+//   256^2 FP64             6.98 / 2.85 / 8.1 us   1000 x 600 FP64    27.8 / 14.9 / 20.4 us
+//   256^2 mixed            4.45 / 3.12 / 8.7      1000 x 600 mixed   16.3 / 12.9 / 14.0
+//   256^2, third absent    8.52 / 2.17 / 8.7      1200^2 FP64        54.2 / 29.0 / 35.6
 // The third phase's terms are 0 * (0 - 0) where no entry of a wavefront and none of its neighbours has
 // that phase, and are left out there (256^2 accelerator call 322 -> 307 us).
 //
@@ -168,7 +169,7 @@ __global__ __launch_bounds__(kTileNT, P == 2 ? (F::kMixed ? 8 : 5) : 4) void dif
   auto self_z = [](const auto &c) {
     A z = c[0] * A(0);
 #pragma unroll
-    for (int p = 1; p < P; ++p) z = __builtin_elementwise_fma(c[p], A(0), z);
+    for (size_t p = 1; p < sizeof(c) / sizeof(c[0]); ++p) z = __builtin_elementwise_fma(c[p], A(0), z);
     return z;
   };
   // a listed cell's place, its neighbours' in the domain and in L, and its depth
@@ -193,26 +194,38 @@ __global__ __launch_bounds__(kTileNT, P == 2 ? (F::kMixed ? 8 : 5) : 4) void dif
     o.gn[3] = gy == ny - 1 ? g + unx - plane : g + unx;
   };
 
-  // the sub-steps, with up to G listed cells per thread
-  auto run = [&](auto entries) {
-    constexpr int G = decltype(entries)::value;
-    A w[G][NF * P], t1[G][P], t2[G][P], cp[G][P], sc[G];
+  // whether a cell of the tile has the third phase (or one of its constants is not finite)
+  auto third_phase = [&]() {
+    bool has = !(dc.D[2] * A(0) == A(0));
+#pragma unroll
+    for (int i = 0; i < 3; ++i) has = has || !((dc.pk[i][2] + dc.pc[i][2]) * A(0) == A(0));
+#pragma unroll
+    for (int k = 0; k < V; ++k)
+      if (t + k * NT < ncells)
+        has = has || ((general >> k) & 1u ? !(pfrac[long(gi[k]) * P + 2] == typename F::T(0))
+                                          : ((phase >> (2 * k)) & 3u) == 2u);
+    return __syncthreads_or(has) != 0;
+  };
+  // the sub-steps, with up to G listed cells per thread and PH phases (those behind are absent)
+  auto run = [&](auto entries, auto phases) {
+    constexpr int G = decltype(entries)::value, PH = decltype(phases)::value;
+    A w[G][NF * PH], t1[G][PH], t2[G][PH], cp[G][PH], sc[G];
     int sdepth[G];
     // saddr: a neighbour's partition in L by face and phase, two places per word.  A bulk neighbour's
     // is its value for the phase it has and 0 for the others (0 * (value - c) would be NaN once the
     // value overflows).
-    static_assert(P * NF % 2 == 0, "two places per word");
-    uint32_t saddr[G][NF * P / 2], sgi[G], present = 0;
+    static_assert(PH * NF % 2 == 0, "two places per word");
+    uint32_t saddr[G][NF * PH / 2], sgi[G], present = 0;
     CompCode sq[G];
     // partition_cell of an entry's value (the division by t1 = 1 of a unit cell changes nothing)
     // whether an entry of the wavefront or a neighbour has the third phase (or its D is not finite)
     bool third = true;
     auto partition = [&](int j) {
 #pragma unroll
-      for (int p = 0; p < P; ++p) {
+      for (int p = 0; p < PH; ++p) {
         if (p == 2 && !third) continue;
         const A v = (sc[j] - t2[j][p]) / t1[j][p];
-        cp[j][p] = ((present >> (j * P + p)) & 1u) ? v : A(0);
+        cp[j][p] = ((present >> (j * PH + p)) & 1u) ? v : A(0);
       }
     };
     bool has = false;
@@ -224,28 +237,28 @@ __global__ __launch_bounds__(kTileNT, P == 2 ? (F::kMixed ? 8 : 5) : 4) void dif
       sgi[j] = 0;
       sc[j] = A(0);
 #pragma unroll
-      for (int q = 0; q < NF * P / 2; ++q) saddr[j][q] = 0;
+      for (int q = 0; q < NF * PH / 2; ++q) saddr[j][q] = 0;
 #pragma unroll
-      for (int p = 0; p < P; ++p) {
+      for (int p = 0; p < PH; ++p) {
         t1[j][p] = A(1);
         t2[j][p] = cp[j][p] = A(0);
       }
 #pragma unroll
-      for (int q = 0; q < NF * P; ++q) w[j][q] = A(0);
+      for (int q = 0; q < NF * PH; ++q) w[j][q] = A(0);
       if (slot < ng) {
         const int idx = list[slot];
         Cell o;
         locate(idx, o);
         sdepth[j] = o.depth;
         sgi[j] = o.g;
-        A ph[P], phn[NF][P];
+        A ph[PH], phn[NF][PH];
 #pragma unroll
-        for (int p = 0; p < P; ++p) ph[p] = A(pfrac[long(o.g) * P + p]);
+        for (int p = 0; p < PH; ++p) ph[p] = A(pfrac[long(o.g) * P + p]);
 #pragma unroll
         for (int f = 0; f < NF; ++f)
 #pragma unroll
-          for (int p = 0; p < P; ++p) phn[f][p] = A(pfrac[long(o.gn[f]) * P + p]);
-        if constexpr (P == 3) {
+          for (int p = 0; p < PH; ++p) phn[f][p] = A(pfrac[long(o.gn[f]) * P + p]);
+        if constexpr (PH == 3) {
           has = has || !(ph[2] == A(0));
 #pragma unroll
           for (int f = 0; f < NF; ++f) has = has || !(phn[f][2] == A(0));
@@ -256,20 +269,20 @@ __global__ __launch_bounds__(kTileNT, P == 2 ? (F::kMixed ? 8 : 5) : 4) void dif
           const int nidx = o.depth > 0 ? idx + o.off[f] : idx;
           const uint32_t s2 = slot_of[nidx];
 #pragma unroll
-          for (int p = 0; p < P; ++p) {
-            const uint32_t a = s2 != 0xffffu      ? uint32_t(CELLS) + s2 * uint32_t(P) + uint32_t(p)
+          for (int p = 0; p < PH; ++p) {
+            const uint32_t a = s2 != 0xffffu      ? uint32_t(CELLS) + s2 * uint32_t(PH) + uint32_t(p)
                                : phn[f][p] > A(0) ? uint32_t(nidx)
                                                   : uint32_t(NONE);
-            const int q = f * P + p;
+            const int q = f * PH + p;
             saddr[j][q >> 1] |= a << (16 * (q & 1));
           }
         }
 #pragma unroll
-        for (int i = 0; i < P; ++i) {
-          if (ph[i] > A(0)) present |= 1u << (j * P + i);
+        for (int i = 0; i < PH; ++i) {
+          if (ph[i] > A(0)) present |= 1u << (j * PH + i);
           A a = ph[0] * dc.pk[i][0], c = ph[0] * dc.pc[i][0];
 #pragma unroll
-          for (int q = 1; q < P; ++q) {
+          for (int q = 1; q < PH; ++q) {
             a += ph[q] * dc.pk[i][q];
             c += ph[q] * dc.pc[i][q];
           }
@@ -279,15 +292,15 @@ __global__ __launch_bounds__(kTileNT, P == 2 ? (F::kMixed ? 8 : 5) : 4) void dif
 #pragma unroll
         for (int f = 0; f < NF; ++f)
 #pragma unroll
-          for (int p = 0; p < P; ++p) w[j][f * P + p] = face_weight<A>(phn[f][p] * ph[p]);
+          for (int p = 0; p < PH; ++p) w[j][f * PH + p] = face_weight<A>(phn[f][p] * ph[p]);
         if constexpr (F::kMixed) sq[j] = comp_unpack(codes[idx]);
         sc[j] = L[idx];
         partition(j);
 #pragma unroll
-        for (int p = 0; p < P; ++p) L[CELLS + slot * P + p] = cp[j][p];
+        for (int p = 0; p < PH; ++p) L[CELLS + slot * PH + p] = cp[j][p];
       }
     }
-    if constexpr (P == 3) third = __any(has) || !(dc.D[2] * A(0) == A(0));
+    if constexpr (PH == 3) third = __any(has) || !(dc.D[2] * A(0) == A(0));
     __syncthreads();
     const int waves_first = t & ~63;  // entries of this wavefront: waves_first + j * NT and on
     for (int s = 1; s <= S; ++s) {
@@ -296,14 +309,14 @@ __global__ __launch_bounds__(kTileNT, P == 2 ? (F::kMixed ? 8 : 5) : 4) void dif
 #pragma unroll
       for (int j = 0; j < G; ++j) {
         if (waves_first + j * NT >= ng) break;  // wave-uniform
-        DelAcc<F, P> acc;
+        DelAcc<F, PH> acc;
         if constexpr (SELF_Z) acc.s[0] = self_z(cp[j]);
 #pragma unroll
         for (int f = 0; f < NF; ++f)
 #pragma unroll
-          for (int p = 0; p < P; ++p) {
+          for (int p = 0; p < PH; ++p) {
             if (p == 2 && !third) continue;  // 0 * (0 - 0)
-            const int q = f * P + p;
+            const int q = f * PH + p;
             const uint32_t a = (saddr[j][q >> 1] >> (16 * (q & 1))) & 0xffffu;
             const A term = w[j][q] * (L[a] - cp[j][p]);
             if (f == 0) acc.first(p, term, dc);
@@ -328,7 +341,7 @@ __global__ __launch_bounds__(kTileNT, P == 2 ? (F::kMixed ? 8 : 5) : 4) void dif
           const int slot = t + j * NT;
           L[list[slot]] = sc[j];
 #pragma unroll
-          for (int p = 0; p < P; ++p) L[CELLS + slot * P + p] = cp[j][p];
+          for (int p = 0; p < PH; ++p) L[CELLS + slot * PH + p] = cp[j][p];
         }
       __syncthreads();
     }
@@ -338,8 +351,58 @@ __global__ __launch_bounds__(kTileNT, P == 2 ? (F::kMixed ? 8 : 5) : 4) void dif
         if (sdepth[j] > 0) codes[list[t + j * NT]] = uint8_t(uint32_t(sq[j]) & 15u);
     }
   };
-  if (__builtin_expect(ng <= NT, 1)) run(std::integral_constant<int, 1>());
-  else run(std::integral_constant<int, V>());
+  using std::integral_constant;
+  if (__builtin_expect(ng <= NT, 1)) {
+    run(integral_constant<int, 1>(), integral_constant<int, P>());
+  } else if (P == 2 || !third_phase()) {
+    run(integral_constant<int, V>(), integral_constant<int, 2>());
+  } else if constexpr (P == 3) {
+    // two entries of three phases do not fit the registers: the full formula from memory, the new
+    // values kept behind the cells until every thread has read
+    for (int s = 1; s <= S; ++s) {
+      const uint32_t key = key_of(s);
+      bulk_step(s, key);
+      for (int i = t; i < ng; i += NT) {
+        const int idx = list[i];
+        Cell o;
+        locate(idx, o);
+        A v = L[idx];
+        if (o.depth >= s) {
+          StencilLoad<F, P, NF> st;
+          st.me.c = typename F::C(v);
+#pragma unroll
+          for (int p = 0; p < P; ++p) st.me.ph[p] = pfrac[long(o.g) * P + p];
+          A z = A(0);
+          if constexpr (SELF_Z) {  // (before the neighbours are loaded: registers)
+            CellPF<A> me;
+            partition_cell<F, P>(st.me, dc, me);
+            z = self_z(me.c);
+            asm volatile("" : "+v"(z));
+          }
+#pragma unroll
+          for (int f = 0; f < NF; ++f) {
+            st.nb[f].c = typename F::C(L[idx + o.off[f]]);
+#pragma unroll
+            for (int p = 0; p < P; ++p) st.nb[f].ph[p] = pfrac[long(o.gn[f]) * P + p];
+          }
+          A del = stencil_del<F, P, NF>(st, dc);
+          if constexpr (SELF_Z) del += z;
+          if constexpr (F::kMixed) {
+            CompCode qo;
+            v = mixed_step(v, del, comp_unpack(codes[idx]), comp_hash(o.g, key), qo);
+            codes[idx] = uint8_t(uint32_t(qo) & 15u);
+          } else {
+            v = v + del;
+          }
+        }
+        L[CELLS + i] = v;
+      }
+      __syncthreads();
+      bulk_write(s);
+      for (int i = t; i < ng; i += NT) L[list[i]] = L[CELLS + i];
+      __syncthreads();
+    }
+  }
 
 #pragma unroll
   for (int k = 0; k < V; ++k)

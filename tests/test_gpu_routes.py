@@ -195,15 +195,17 @@ def test_larger_plane(P, form, params):  # noqa: F811
     print(f"[gpu] plane {shape} P={P} form={form}", flush=True)
     rng = np.random.default_rng(43)
     sub.check(shape, 0, P, form, sub.sparse_state(rng, *shape, P), params, (1, 14))
-    sub.check(shape, 0, P, form, dense_state(rng, 363 * 367, P), params, (7,))
+    for phases in range(2, P + 1):
+        sub.check(shape, 0, P, form, dense_state(rng, 363 * 367, phases), params, (7,))
 
 
 @pytest.mark.parametrize("shape", [(64, 33, 1), (37, 20, 11), (64, 12, 16), (363, 367, 1), (2, 200000, 1),
                                    (1300, 1161, 1)])
 @pytest.mark.parametrize("loops", [1, 2])
 def test_accelerator_calls_against_the_oracle(shape, loops, params):  # noqa: F811
-    """Both accelerator calls, which share kernels, against the oracle: tiles, the one-launch kernel, and
-    planes that take neither size of tile (narrow, and above 1.5 M cells)."""
+    """Both accelerator calls, which share kernels, against the oracle, with few and with all cells
+    listed: tiles, the one-launch kernel, and planes that take neither size of tile (narrow, and above
+    1.5 M cells)."""
     print(f"[gpu] accelerator calls {shape} loops={loops}", flush=True)
     stream = torch.cuda.current_stream().cuda_stream
     q = PfParams.from_buffer_copy(params)
@@ -212,7 +214,8 @@ def test_accelerator_calls_against_the_oracle(shape, loops, params):  # noqa: F8
     pk = np.array([[q.part_k[0][i][j] for j in range(3)] for i in range(3)]).T.reshape(-1).copy()
     pc = np.array([[q.part_c[0][i][j] for j in range(3)] for i in range(3)]).T.reshape(-1).copy()
     dt = (loops - 0.1) * (q.dx * q.dx / D.max() / (3 if shape[2] > 1 else 2) * float(np.float32(0.2)))
-    state = sub.sparse_state(np.random.default_rng(44), *shape, 3)
+    rng = np.random.default_rng(44)
+    state = sub.sparse_state(rng, *shape, 3) if loops == 1 else dense_state(rng, int(np.prod(shape)), 2)
     o = oracle.OracleDomain(*shape, 4, 1)
     o.set_params(oracle.as_orc_params(q))
     o.set_state(*state)
