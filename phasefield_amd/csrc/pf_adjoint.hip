@@ -84,14 +84,14 @@ __device__ inline void part_deriv(double c, const double *ph, const DiffConsts<d
 }
 
 // sum of one double over the workgroup (256 lanes = 4 wavefronts), added to acc[blockIdx.x]
-__device__ inline void block_accumulate(double v, double *__restrict__ acc) {
+__device__ inline void block_accumulate(double v, double *__restrict__ acc, unsigned at) {
   __shared__ double part[4];
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0) part[wave] = v;
   __syncthreads();
-  if (threadIdx.x == 0) acc[blockIdx.x] += (part[0] + part[1]) + (part[2] + part[3]);
+  if (threadIdx.x == 0) acc[at] += (part[0] + part[1]) + (part[2] + part[3]);
 }
 
 // Reverse of one sub-step: lam_out = dL/dc^s given lam_in = dL/dc^{s+1} and c^s; accumulates
@@ -201,7 +201,7 @@ __global__ __launch_bounds__(256) void adj_diffuse_kernel(
       dD0 = adj_cell<P, NF, NOFLUX>(j, c, pf, lam_in, lam_out, lam_pf, dc, nx, ny, nz);
     }
   }
-  block_accumulate(dD0, accD);
+  block_accumulate(dD0, accD, blockIdx.x);
 }
 
 // Split form: the listed cells (flag 0 after adj_list_flag_kernel: interface cells and bulk cells
@@ -219,12 +219,12 @@ __global__ __launch_bounds__(256) void adj_general_kernel(
   double dD0 = 0.0;
   for (int k = blockIdx.x * 256 + threadIdx.x; k < n; k += gridDim.x * 256)
     dD0 += adj_cell<P, NF, NOFLUX>(list[k], c, pf, lam_in, lam_out, lam_pf, dc, nx, ny, nz);
-  block_accumulate(dD0, accD);
+  block_accumulate(dD0, accD, blockIdx.x);
 }
 
 // The reverse sub-step in one launch, where the forward one is (pf_diffuse_direct.hip): the listed cells by
-// the first workgroups, the bulk cells of phases other than 1 by the others, the same update with lam
-// for c.  128^3, per reverse sub-step: marching kernel and listed pass 23.7 us, one launch 15.6 us, and
+// the first (and last) workgroups, the bulk cells of phases other than 1 by the others, the same update
+// with lam for c.  128^3, per reverse sub-step: marching kernel and listed pass 23.7 us, one launch 15.6 us, and
 // 14.3 us with a listed cell's loads issued together (60 x 50 x 40, whole runs: 6.0 -> 4.9 ms).
 template <int P, bool NOFLUX, int V, int U>
 __global__ __launch_bounds__(256) void adj_direct_kernel(
@@ -233,19 +233,21 @@ __global__ __launch_bounds__(256) void adj_direct_kernel(
     double *__restrict__ lam_out, double *__restrict__ lam_pf, double *__restrict__ accD,
     const DiffConsts<double> dc, const DirectGeom geo) {
   const int b = blockIdx.x;
-  if (b < geo.nlist) {
+  const int bulk = b - geo.nlist;
+  if (__builtin_expect(unsigned(bulk) >= unsigned(geo.nbulk), 0)) {
+    const int group = bulk < 0 ? b : b - geo.nbulk;
     // the first entry is read along with the list's length (the list has room for every cell)
-    const int stride = geo.nlist * 256;
-    int k = b * 256 + threadIdx.x;
+    const uint32_t stride = uint32_t(geo.nlist + geo.nmore) * 256u;
+    uint32_t k = uint32_t(group) * 256u + threadIdx.x;
     int e = list[min(long(k), long(geo.nx) * geo.ny * geo.nz - 1)];
-    const int n = *count;
+    const uint32_t n = uint32_t(*count);
     double dD0 = 0.0;
     for (; k < n; k += stride, e = k < n ? list[k] : 0)
       dD0 += adj_cell<P, 6, NOFLUX>(e, c, pf, lam_in, lam_out, lam_pf, dc, geo.nx, geo.ny, geo.nz);
-    block_accumulate(dD0, accD);
+    block_accumulate(dD0, accD, group);
     return;
   }
-  direct_bulk<FormF64, P, NOFLUX, V, U>(lam_in, lam_out, packed, dc, geo, b - geo.nlist);
+  direct_bulk<FormF64, P, NOFLUX, V, U>(lam_in, lam_out, packed, dc, geo, bulk);
 }
 
 // bulk flags of phase 1 -> 0, so those cells join the listed pass
@@ -830,9 +832,10 @@ template <int K, int P, int NF, bool NOF> struct Adj {
             auto go = [&](auto run) {
               constexpr int V = decltype(run)::value;
               set_runs(g, false, V, 2);
-              hipLaunchKernelGGL((adj_direct_kernel<P, NOF, V, 2>), dim3(unsigned(g.nlist + g.nbulk)),
-                                 dim3(256), 0, st, sd.csub + size_t(N) * s, sd.pf_new, packed, alist,
-                                 ablock + nl, lam_c, lam_c2, lam_pf, accD, dc, g);
+              // (its partials of dL/dD, one per workgroup of the list: at most gb)
+              hipLaunchKernelGGL((adj_direct_kernel<P, NOF, V, 2>),
+                                 dim3(unsigned(g.nlist + g.nbulk + g.nmore)), dim3(256), 0, st,
+                                 sd.csub + size_t(N) * s, sd.pf_new, packed, alist, ablock + nl, lam_c, lam_c2, lam_pf, accD, dc, g);
             };
             if (vec) go(std::integral_constant<int, 2>());
             else go(std::integral_constant<int, 1>());

@@ -6,7 +6,8 @@
 
 namespace pfamd {
 
-// n / d and n % d for 0 <= n < 2^31 by one multiplication: with s = ceil(log2 d) and
+// n / d and n % d for 0 <= n < 2^31 by one multiplication with the rounded-up reciprocal (Granlund and
+// Montgomery's division by invariant integers): with s = ceil(log2 d) and
 // m = ceil(2^(31+s) / d) < 2^32 the error m * d - 2^(31+s) is below 2^s, so n * error stays below
 // 2^(31+s) and the quotient is exact.
 struct FastDiv {
@@ -23,12 +24,13 @@ struct FastDiv {
 };
 
 struct DirectGeom {
+  int nlist;     // workgroups of the listed cells, ahead of the others
+  int nbulk;     // workgroups of the bulk cells
+  int nmore;     // workgroups of the listed cells behind the others
+  int flip;      // walk the bulk cells from the last to the first
   int nx, ny, nz;
   FastDiv row;   // runs of V cells per row (mixed, V == 1: cells per row)
   FastDiv rows;  // rows per plane
-  int nlist;     // workgroups of the listed cells, ahead of the others
-  int nbulk;     // workgroups of the bulk cells
-  bool flip;     // walk the bulk cells from the last to the first
 };
 
 // One sub-step: the bulk cells of every phase in runs of V cells times U planes per thread, the
@@ -50,10 +52,16 @@ inline DirectGeom direct_geometry(int nx, int ny, int nz, bool flip) {
   g.ny = ny;
   g.nz = nz;
   g.flip = flip;
-  // the listed part: one entry per thread up to a sixteenth of the cells (a round of entries is a
+  // The listed part: one entry per thread up to a sixteenth of the cells (a round of entries is a
   // chain of three memory latencies and the full formula), at least 64 workgroups where the domain
-  // has that many (40 x 24 x 16 with 4 workgroups: 11.0 us, with 60: 4.3)
+  // has that many (40 x 24 x 16 with 4 workgroups: 11.0 us, with 60: 4.3).  Domains of up to 2^20 cells
+  // have seven times as many again behind the bulk cells, which end at once where the list is
+  // short: 64^3 FP64 with every cell listed 11.8 us, 37.1 without them (18.2 in a listed pass of its own),
+  // with 3 % listed 4.9 either way.  (The bulk workgroups going on with the list instead: every cell
+  // listed 16.4, and 1.5-3.5 % on short lists at 128^3.)  Never more than one entry per thread,
+  // so there are at most (n + 255) / 256 of them.
   g.nlist = int(std::min<long>(1024, std::max<long>((n + 4095) / 4096, std::min<long>(64, (n + 255) / 256))));
+  g.nmore = n <= (1L << 20) ? int(std::min<long>(7L * g.nlist, (n + 255) / 256 - g.nlist)) : 0;
   return g;
 }
 // runs of V cells times U planes; pairs: byte pairs in storage order instead
@@ -83,8 +91,9 @@ hipError_t launch_direct(hipStream_t stream, const typename F::C *cin, typename 
   auto go = [&](auto v, auto u) {
     constexpr int V = decltype(v)::value, U = decltype(u)::value;
     set_runs(g, F::kMixed && V == 1, V, U);
-    hipLaunchKernelGGL((diffuse_direct_kernel<F, P, NOF, V, U>), dim3(unsigned(g.nlist + g.nbulk)),
-                       dim3(256), 0, stream, cin, cout, pfrac, packed, list, count, dc, g);
+    hipLaunchKernelGGL((diffuse_direct_kernel<F, P, NOF, V, U>),
+                       dim3(unsigned(g.nlist + g.nbulk + g.nmore)), dim3(256), 0, stream, cin, cout,
+                       pfrac, packed, list, count, dc, g);
   };
   using std::integral_constant;
   if constexpr (F::kMixed) {

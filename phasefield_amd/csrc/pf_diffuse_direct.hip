@@ -4,9 +4,9 @@
 //
 // Up to 128^3 a sub-step is bound by the launches and by one round of memory latency, not by bytes
 // (an empty launch takes 1.6 us, a pass over 64^3 cells 2.8 us), so the bulk cells and the listed
-// cells share one launch: the first workgroups take the list, the others the bulk cells, and each
-// cell is written by exactly one of them (a bulk thread skips what the flags list).  The bulk part
-// keeps nothing in LDS and has no loop: every load of a thread is issued before the first is used,
+// cells share one launch: the first (and, for long lists, the last) workgroups take the list, the
+// others the bulk cells, and each cell is written by exactly one of them (a bulk thread skips what the
+// flags list).  The bulk part keeps nothing in LDS and has no loop: every load of a thread is issued before the first is used,
 // and each XCD takes a contiguous range of the domain, so the y and z neighbours come from its L2
 // (128^3 FP64 pass alone: 6.6 us with contiguous ranges, 7.3 us in launch order, 4.1 us for a plain
 // copy).  Flags are read as two bits per cell.
@@ -67,12 +67,15 @@ __global__ __launch_bounds__(256) void diffuse_direct_kernel(
   const long n = long(plane) * nz;
   const int b = blockIdx.x;
 
-  if (b < geo.nlist) {
+  const int bulk = b - geo.nlist;
+  if (__builtin_expect(unsigned(bulk) >= unsigned(geo.nbulk), 0)) {
+    const int group = bulk < 0 ? b : b - geo.nbulk;
     // the first entry is read along with the list's length (the list has room for every cell)
-    const int stride = geo.nlist * 256;
-    int k = b * 256 + threadIdx.x;
+    // (unsigned: an index below 2^31 and a round of threads)
+    const uint32_t stride = uint32_t(geo.nlist + geo.nmore) * 256u;
+    uint32_t k = uint32_t(group) * 256u + threadIdx.x;
     int e = list[min(long(k), n - 1)];
-    const int m = *count;
+    const uint32_t m = uint32_t(*count);
     for (; k < m; k += stride, e = k < m ? list[k] : 0) {
       if constexpr (F::kMixed) {
         // a byte pair (ListOrder::pairs): both cells are computed and stored, with their code byte;
@@ -104,7 +107,7 @@ __global__ __launch_bounds__(256) void diffuse_direct_kernel(
     return;
   }
 
-  direct_bulk<F, P, NOFLUX, V, U>(cin, cout, packed, dc, geo, b - geo.nlist);
+  direct_bulk<F, P, NOFLUX, V, U>(cin, cout, packed, dc, geo, bulk);
 }
 
 #define PF_INST_DIRECT(F, P, NOF, V, U)                                                       \

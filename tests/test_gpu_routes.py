@@ -150,18 +150,21 @@ def dense_state(rng, n, P):
     return ids.reshape(-1), val.reshape(-1), phase.reshape(-1), 0.02 + 0.8 * rng.random(n)
 
 
+LONG = [((40, 36, 30), 0, 2), ((65, 61, 39), 1, 3), ((104, 102, 100), 0, 2)]
+
+
 @pytest.mark.parametrize("form", FORMS)
-@pytest.mark.parametrize("shape,bc,P", [((40, 36, 30), 0, 2), ((41, 37, 29), 1, 3)])
+@pytest.mark.parametrize("shape,bc,P", LONG)
 def test_more_listed_cells_than_threads(shape, bc, P, form, params):  # noqa: F811
-    """64 workgroups take the list of the one-launch kernel here: 16384 entries at a time, of 43 200
-    cells and of half as many byte pairs."""
+    """Lists that go on behind the one-launch kernel's first workgroups, 16384 entries here: in the
+    workgroups behind the bulk cells, in a second round of both (above 131072 entries), and, above 2^20
+    cells, in rounds of the first alone; cells and byte pairs."""
     print(f"[gpu] long list {shape} bc={bc} P={P} form={form}", flush=True)
     n = int(np.prod(shape))
-    assert n // 2 > 16384
     sub.check(shape, bc, P, form, dense_state(np.random.default_rng(41), n, P), params, (1, 2))
 
 
-@pytest.mark.parametrize("shape,bc,P", [((40, 36, 30), 0, 2), ((41, 37, 29), 1, 3)])
+@pytest.mark.parametrize("shape,bc,P", LONG)
 def test_adjoint_more_listed_cells_than_threads(monkeypatch, shape, bc, P, params):  # noqa: F811
     """The reverse sub-step over the same lists, in one launch and in the separate listed pass: d_conc0
     by the same operations, the sums over the cells in another order."""
