@@ -4,8 +4,9 @@
 // hipMalloc).  The caller passes value_phase and total_conc in device memory and a stream; the
 // sub-steps run asynchronously on that stream with the kernels of the handle API: the bulk flags and
 // the list once per call, then the tile kernel (one plane, several sub-steps per launch) or the
-// one-launch sub-step (3D).  Before, every sub-step ran the full formula for every cell: 256^2 1.19 ms
-// a call of 200 sub-steps, 128^3 8.5 ms.
+// one-launch sub-step (3D; large domains the LDS-tiled full formula where no phase's partition is the
+// identity).  Before, every sub-step ran the full formula for every cell: 256^2 1.19 ms a call of 200
+// sub-steps, 128^3 8.5 ms.
 //
 // What a call needs besides the caller's arrays is in file-scope device arrays with room for
 // kNoAllocMaxCells cells (28.5 MiB), which every GPU the library is loaded on holds until the process
@@ -141,17 +142,35 @@ extern "C" int pf_gpu_diffusion_solver_noalloc(const double *hdiffusivity,
   unsigned mask = 0;
   for (int p = 0; p < 3; ++p)
     if (dc.pk[p][p] == 1.0 && dc.pc[p][p] == 0.0) mask |= 1u << (p + 1);
-  // six faces always, as Diff3D sums them (gpu_solver.cpp:160-188)
-  e = launch_classify<double, 3, 6, false>(s, pf, buf.unit, buf.flag, x, y, z, N, mask, buf.count);
+  TileGeom tile;
+  const bool tiles = z == 1 && tile_geometry(x, y, 1, false, num_loop, nullptr, tile);
+  // (six faces always, as Diff3D sums them, gpu_solver.cpp:160-188)
+  // No phase has a reduced form: every cell takes the full formula, which the LDS-tiled kernel shares
+  // between neighbours (128^3, 200 sub-steps: 8.59 ms, 13.71 with every cell listed).  Its columns leave a
+  // smaller domain's latency bare (60^3 8.18 ms, 2.88 with every cell listed).
+  const bool full = !mask && !tiles && N > (1L << 20);
+  if (!full)
+    e = launch_classify<double, 3, 6, false>(s, pf, buf.unit, buf.flag, x, y, z, N, mask, buf.count);
   if (e != hipSuccess)
     return set_global_error(PF_ERR_HIP, std::string("pf_gpu_diffusion_solver_noalloc: launch: ") +
                                             hipGetErrorString(e));
-  TileGeom tile;
-  if (z == 1 && tile_geometry(x, y, 1, false, num_loop, nullptr, tile)) {
+  if (tiles) {
     for (int left = num_loop; left > 0; left -= tile.steps) {
       (void)tile_geometry(x, y, 1, false, left, nullptr, tile);
       hipLaunchKernelGGL((diffuse_tile_kernel<FormF64, 3, true>), dim3(unsigned(tile.nblocks)),
                          dim3(kTileNT), 0, s, a, b, pf, buf.flag, dc, tile, N, 0u, 0);
+      std::swap(a, b);
+    }
+  } else if (full) {
+    // 64 x kDiffTY columns, z split into chunks of >= 16 planes until about 2048 workgroups.
+    const int tiles_x = (x + 63) / 64, tiles_y = (y + kDiffTY - 1) / kDiffTY;
+    const long columns = long(tiles_x) * tiles_y;
+    const long nzc = std::max(1L, std::min<long>(z, (2048 + columns - 1) / columns));
+    const int zc = std::max(int((z + nzc - 1) / nzc), std::min(z, 16));
+    const int nblocks = int(columns * ((z + zc - 1) / zc));
+    for (int it = 0; it < num_loop; ++it) {
+      hipLaunchKernelGGL((diffuse_kernel<FormF64, 3, 6, false, kDiffTY>), dim3(unsigned(nblocks)),
+                         dim3(64, kDiffTY + 3), 0, s, a, b, pf, dc, x, y, z, zc, tiles_x, tiles_y, nblocks);
       std::swap(a, b);
     }
   } else {
