@@ -138,10 +138,16 @@ extern "C" int pf_gpu_diffusion_solver_noalloc(const double *hdiffusivity,
   dc.r = dt / num_loop / (dx * dx);
   const double *pf = dvalue_phase;
   double *a = dtotal_conc, *b = buf.conc;
-  // phases whose bulk cells take the reduced form: identity partition
+  // Phases whose bulk cells take the reduced form: identity partition.  None where a constant is not
+  // finite: the full formula multiplies it by the zeros of absent phases, which the reduced form drops.
+  bool finite = true;
+  for (int i = 0; i < 3; ++i) {
+    finite = finite && std::isfinite(dc.D[i]);
+    for (int j = 0; j < 3; ++j) finite = finite && std::isfinite(dc.pk[i][j]) && std::isfinite(dc.pc[i][j]);
+  }
   unsigned mask = 0;
   for (int p = 0; p < 3; ++p)
-    if (dc.pk[p][p] == 1.0 && dc.pc[p][p] == 0.0) mask |= 1u << (p + 1);
+    if (finite && dc.pk[p][p] == 1.0 && dc.pc[p][p] == 0.0) mask |= 1u << (p + 1);
   TileGeom tile;
   const bool tiles = z == 1 && tile_geometry(x, y, 1, false, num_loop, nullptr, tile);
   // (six faces always, as Diff3D sums them, gpu_solver.cpp:160-188)

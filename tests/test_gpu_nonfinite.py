@@ -100,3 +100,39 @@ def test_overflowed_partition_of_a_plane_with_six_faces(loops, params):
     assert rc == 0, lib().pf_last_error(None)
     assert different(dconc.cpu().numpy(), want) == []
     assert different(host, want) == []
+
+
+@pytest.mark.parametrize("constant", ["D", "pk", "pc"])
+@pytest.mark.parametrize("shape", [(40, 24, 1), (41, 24, 16)])
+def test_nonfinite_constant_of_an_absent_phase(shape, constant, params):
+    """The allocation-free call: a phase that no cell has, with a constant that is not finite, makes every
+    cell NaN (0 * NaN), bulk cells too."""
+    print(f"[gpu] non-finite {constant} {shape}", flush=True)
+    nx, ny, nz = shape
+    planes = [ferrite(nx, ny, [10 + nx * 10]) for _ in range(nz)]
+    ids, val, phase, conc = (np.concatenate(a) for a in zip(*planes))
+    q = PfParams.from_buffer_copy(params)
+    q.dims = 3 if nz > 1 else 2
+    D = np.array([q.diffusivity[0][i] for i in range(3)])
+    dt = 2.9 * (q.dx * q.dx / D.max() / q.dims * float(np.float32(0.2)))
+    if constant == "D":
+        q.diffusivity[0][2] = D[2] = np.nan
+    elif constant == "pk":
+        q.part_k[0][1][2] = np.inf
+    else:
+        q.part_c[0][1][2] = np.inf
+    pk = np.array([[q.part_k[0][i][j] for j in range(3)] for i in range(3)]).T.reshape(-1).copy()
+    pc = np.array([[q.part_c[0][i][j] for j in range(3)] for i in range(3)]).T.reshape(-1).copy()
+    o = oracle.OracleDomain(nx, ny, nz, 4, 1)
+    o.set_params(oracle.as_orc_params(q))
+    o.set_state(ids, val, phase, conc)
+    o.diffuse_factor(0, 3, dt / 3 / (q.dx * q.dx))
+    want = o.get_state()["conc"]
+    assert np.isnan(want).all()
+    dphase = torch.from_numpy(phase).to("cuda:0")
+    dconc = torch.from_numpy(conc).to("cuda:0")
+    ptr = [a.ctypes.data_as(ctypes.POINTER(ctypes.c_double)) for a in (D, pk, pc)]
+    rc = lib().pf_gpu_diffusion_solver_noalloc(*ptr, dphase.data_ptr(), dconc.data_ptr(), nx, ny, nz, dt,
+                                               q.dx, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib().pf_last_error(None)
+    assert different(dconc.cpu().numpy(), want) == []
