@@ -35,8 +35,9 @@ struct DirectGeom {
 
 // One sub-step: the bulk cells of every phase in runs of V cells times U planes per thread, the
 // listed cells (flag 0; mixed: the byte pairs that hold one) by the first workgroups.  `packed`: the
-// bulk flags, two bits per cell (general_count_kernel).
-template <class F, int P, bool NOFLUX, int V, int U>
+// bulk flags, two bits per cell (general_count_kernel).  MORE: geo.nmore > 0 (a kernel of its own: the test
+// for workgroups behind the bulk cells costs the allocation-free call at 128^3 1.5 %).
+template <class F, int P, bool NOFLUX, int V, int U, bool MORE>
 __global__ void diffuse_direct_kernel(const typename F::C *__restrict__ cin,
                                       typename F::C *__restrict__ cout,
                                       const typename F::T *__restrict__ pfrac,
@@ -91,9 +92,10 @@ hipError_t launch_direct(hipStream_t stream, const typename F::C *cin, typename 
   auto go = [&](auto v, auto u) {
     constexpr int V = decltype(v)::value, U = decltype(u)::value;
     set_runs(g, F::kMixed && V == 1, V, U);
-    hipLaunchKernelGGL((diffuse_direct_kernel<F, P, NOF, V, U>),
-                       dim3(unsigned(g.nlist + g.nbulk + g.nmore)), dim3(256), 0, stream, cin, cout,
-                       pfrac, packed, list, count, dc, g);
+    auto kernel = g.nmore > 0 ? diffuse_direct_kernel<F, P, NOF, V, U, true>
+                              : diffuse_direct_kernel<F, P, NOF, V, U, false>;
+    hipLaunchKernelGGL(kernel, dim3(unsigned(g.nlist + g.nbulk + g.nmore)), dim3(256), 0, stream, cin,
+                       cout, pfrac, packed, list, count, dc, g);
   };
   using std::integral_constant;
   if constexpr (F::kMixed) {

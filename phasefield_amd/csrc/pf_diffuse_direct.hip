@@ -55,7 +55,7 @@ __device__ inline float bulk_del(const StencilLoad<FormMixed, P, 6> &s, const Di
 
 }  // namespace
 
-template <class F, int P, bool NOFLUX, int V, int U>
+template <class F, int P, bool NOFLUX, int V, int U, bool MORE>
 __global__ __launch_bounds__(256) void diffuse_direct_kernel(
     const typename F::C *__restrict__ cin, typename F::C *__restrict__ cout,
     const typename F::T *__restrict__ pfrac, const uint32_t *__restrict__ packed,
@@ -68,11 +68,11 @@ __global__ __launch_bounds__(256) void diffuse_direct_kernel(
   const int b = blockIdx.x;
 
   const int bulk = b - geo.nlist;
-  if (__builtin_expect(unsigned(bulk) >= unsigned(geo.nbulk), 0)) {
+  if (MORE ? __builtin_expect(unsigned(bulk) >= unsigned(geo.nbulk), 0) : bulk < 0) {
     const int group = bulk < 0 ? b : b - geo.nbulk;
     // the first entry is read along with the list's length (the list has room for every cell)
     // (unsigned: an index below 2^31 and a round of threads)
-    const uint32_t stride = uint32_t(geo.nlist + geo.nmore) * 256u;
+    const uint32_t stride = uint32_t(geo.nlist + (MORE ? geo.nmore : 0)) * 256u;
     uint32_t k = uint32_t(group) * 256u + threadIdx.x;
     int e = list[min(long(k), n - 1)];
     const uint32_t m = uint32_t(*count);
@@ -110,13 +110,15 @@ __global__ __launch_bounds__(256) void diffuse_direct_kernel(
   direct_bulk<F, P, NOFLUX, V, U>(cin, cout, packed, dc, geo, bulk);
 }
 
-#define PF_INST_DIRECT(F, P, NOF, V, U)                                                       \
-  template __global__ void diffuse_direct_kernel<F, P, NOF, V, U>(                            \
+#define PF_INST_DIRECT(F, P, NOF, V, U, MORE)                                                 \
+  template __global__ void diffuse_direct_kernel<F, P, NOF, V, U, MORE>(                      \
       const F::C *, F::C *, const F::T *, const uint32_t *, const int *, const int *,          \
       const DiffConsts<F::A>, DirectGeom);
-#define PF_INST_DIRECT_NOF(F, P, V, U) \
-  PF_INST_DIRECT(F, P, false, V, U)    \
-  PF_INST_DIRECT(F, P, true, V, U)
+#define PF_INST_DIRECT_NOF(F, P, V, U)     \
+  PF_INST_DIRECT(F, P, false, V, U, false) \
+  PF_INST_DIRECT(F, P, false, V, U, true)  \
+  PF_INST_DIRECT(F, P, true, V, U, false)  \
+  PF_INST_DIRECT(F, P, true, V, U, true)
 #define PF_INST_DIRECT_P(P)            \
   PF_INST_DIRECT_NOF(FormF64, P, 1, 2)   \
   PF_INST_DIRECT_NOF(FormF64, P, 2, 2)   \
