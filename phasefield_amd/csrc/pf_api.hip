@@ -561,14 +561,21 @@ bool default_diffusion(const pf_handle *h) {
          h->diff_zchunk_override == 0;
 }
 // Whether they run as one launch of the direct kernel: rows the marching kernel does not take, and
-// domains whose two concentration buffers are at most half of the memory-side cache.  Per step, one
+// domains whose two concentration buffers are at most half of the 256 MB memory-side cache.  Per step, one
 // domain on the GPU / each of three in turn, marching + listed pass against the direct kernel:
-//   128^3 FP64 (34 MB)    3.37 / 2.30 ms against 1.88 / 1.55
-//   192^3 mixed (64 MB)   6.36 / 3.95    against 3.67 / 3.05
-//   192^3 FP64 (113 MB)   8.61 / 5.75    against 4.80 / 6.18
+//   128^3 FP64 (34 MB)    3.27 / 2.17 ms against 2.05 / 1.61
+//   160^3 FP64 (66 MB)    6.06 / 4.20    against 3.36 / 2.90
+//   176^3 FP64 (87 MB)    6.54 / 4.82    against 4.20 / 4.98
+//   192^3 FP64 (113 MB)   8.45 / 6.66    against 5.08 / 7.22
+//   200^3 FP64 (128 MB)   8.95 / 7.08    against 5.78 / 8.57
+//   192^3 mixed (64 MB)   6.49 / 3.96    against 3.58 / 2.99
+//   240^3 mixed (124 MB)  9.01 / 7.03    against 5.87 / 7.72
 //   224^3 FP64 (180 MB)  11.29 / 8.56    against 7.31 / 10.01
 //   256^3 FP64 (268 MB)  14.29 / 12.39   against 12.92 / 14.58
-// Beyond half of the cache a second domain's passes push the first one's out between two sub-steps.
+// One domain alone gains as long as its buffers fit the cache; where several share it, one's passes push
+// the others' out between two sub-steps, and from about 80 MB on the direct kernel, which reads every
+// neighbour from the caches, loses.  The line is set for one domain (35 % and more up to it) at the price
+// of at most 21 % where three take turns.
 bool use_direct(const pf_handle *h, int nf) {
   if (!h->diff_direct || nf != 6 || h->d.nz == 1 || !default_diffusion(h)) return false;
   const bool march = is_mixed(h) ? use_march<FormMixed>(h) : use_march<FormF64>(h);
