@@ -1,4 +1,4 @@
-"""GPU: diffusion sub-steps of planes in which a concentration, or a phase's share of it, has overflowed:
+"""GPU: diffusion sub-steps in which a concentration, a phase's share of it or a constant is not finite:
 infinities and NaN stand where the full-formula kernel has them.  There an absent phase's partition is
 0; the oracle divides for absent phases too, so its 0 * (inf - c) is NaN where the kernels have 0."""
 from __future__ import annotations
